@@ -201,6 +201,28 @@ def test_long_prefill_chunks(gpu, models):
         assert np.max(np.abs(got - ref.forward(toks, 0))) < LOGIT_TOL
 
 
+@pytest.mark.parametrize("name", ["qwen2", "qwen3_rope_half"])
+@pytest.mark.parametrize("n", [9, 16, 17, 33, 65, 129, 300])
+def test_prefill_tile_cuts_match_oracle(gpu, tmp_path, name, n):
+    """The prefill tile GEMM's cuts around their edges: 16 / 32 / 64 / 128 tokens per workgroup, K in
+    slices whose partial outputs the next kernel adds (qwen2: biases added once, gate | up slices; half
+    RoPE: a q|k|v reader that takes no slices). Every cut's logits at the gate against the oracle, or,
+    for the half RoPE that the oracle's model does not have, against the same tokens decoded one by one."""
+    cfg = configs.tiny("qwen2" if name == "qwen2" else "qwen3", tie=False, hidden=1024, inter=2048)
+    if name != "qwen2":
+        cfg = dict(cfg, partial_rotary_factor=0.5)
+    mlxr.synth_write(cfg, seed=n, directory=str(tmp_path))
+    with mlxr.Transformer(str(tmp_path), context_length=1024) as m:
+        toks = prompt(n, m.vocab_size, seed=n)
+        if name == "qwen2":
+            exp = oracle.Model(str(tmp_path), m.max_seq).forward(toks, 0)
+        else:
+            for i in range(n):
+                exp = m.forward(toks[i:i + 1], i)
+        got = m.forward(toks, 0)
+        assert np.max(np.abs(got - exp)) < LOGIT_TOL
+
+
 def test_sparse_full_budget_is_bit_identical(gpu, models):
     """sparseDecodeWithFullBudgetIsBitIdentical (ModelTests.swift:155-182)."""
     d = models["qwen3"]
