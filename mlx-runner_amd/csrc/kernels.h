@@ -56,19 +56,18 @@ struct QGemmArgs {
     const float* x = nullptr; int x_stride = 0;
     float* y = nullptr; int y_stride = 0;
     // pre-pass scratch: hi and lo (T*K 16-bit each), group sums (qgemm_gsum_floats), the rows' inverse
-    // scales (T floats), lo-nonzero flags (T ints) and the repacked scales and biases
-    // (qgemm_scale_halves 16-bit words)
+    // scales (T floats), lo-nonzero flags (T ints) and room for repacked scales and biases
+    // (qgemm_scale_halves 16-bit words; used where a row's groups are odd in number)
     uint16_t* xbf = nullptr; uint16_t* xlo = nullptr; float* xgs = nullptr; float* xsc = nullptr; int* xnz = nullptr;
     uint16_t* wsb = nullptr;
     bool x_ready = false;                 // the scratch already holds this x (same K and gs): skip the pre-pass
-    // optional scratch for the split over K when the grid is under one round:
-    // QGEMM_SPLIT_FLOATS floats, zero before first use (its tile counters return to zero)
+    // optional scratch for K slices on workgroups of their own: QGEMM_SPLIT_FLOATS floats, zero before
+    // first use (its tile counters return to zero)
     float* split = nullptr; size_t split_floats = 0;
 };
-// tile counters for up to 256 tiles, then at most 256 partial 128 x 256 tiles (slices x tiles stay
-// within one workgroup per CU of a 256-CU device)
-constexpr size_t QGEMM_SPLIT_TILES = 256;
-constexpr size_t QGEMM_SPLIT_FLOATS = QGEMM_SPLIT_TILES + QGEMM_SPLIT_TILES * 128 * 256;
+// tile counters, then the slices' partial tiles (512 of 128 x 256, or as many smaller ones as fit)
+constexpr size_t QGEMM_SPLIT_TILES = 4096, QGEMM_SPLIT_PART = 512 * 128 * 256;
+constexpr size_t QGEMM_SPLIT_FLOATS = QGEMM_SPLIT_TILES + QGEMM_SPLIT_PART;
 hipError_t launch_qgemm(const QGemmArgs& a, hipStream_t s);
 size_t qgemm_gsum_floats(int T, int K, int gs);
 bool qgemm_supported(int K, int gs);   // K % 64 == 0, gs 32 / 64 / 128

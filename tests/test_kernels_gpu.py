@@ -166,6 +166,42 @@ def test_qgemm_prefill_tiles(gpu, bits, gs):
         assert max_rel_err(qgemm(gpu, fx, x), fx.oracle(oracle).matmul_f64(x)) < TOL, st
 
 
+@pytest.mark.parametrize("gs", [32, 64, 128])
+@pytest.mark.parametrize("bits", [2, 3, 4, 5, 6, 8])
+def test_qgemm_cuts(gpu, bits, gs):
+    """The MLX-layout GEMM's tile shapes and K slices around their edges (32 / 64 / 128 tokens, 128 / 256
+    rows; 2176 inputs: two slices, a group count that is odd at gs 128; 8320: eight, of uneven length):
+    each T against the fp64 product at the gate, its rows bit-identical to those of the largest T."""
+    for O, K in ((300, 2176), (129, 8320)):
+        fx = QuantFixture(O, K, bits, gs, seed=bits + gs, fast=True)
+        x = np.random.default_rng(gs + bits).uniform(-1, 1, (200, K)).astype(np.float32)
+        ref = fx.oracle(oracle).matmul_f64(x)
+        full = qgemm(gpu, fx, x)
+        assert max_rel_err(full, ref) < TOL, (O, K)
+        for T in (9, 32, 33, 65, 129):
+            assert np.array_equal(qgemm(gpu, fx, x[:T]).view(np.uint32), full[:T].view(np.uint32)), (T, O, K)
+
+
+def test_qgemm_pointer_alignment(gpu):
+    """Codes at a 4-byte and scales / biases at a 2-byte boundary (the smallest that their types give)."""
+    O, K, bits, gs, T = 70, 1024, 6, 64, 20
+    fx = QuantFixture(O, K, bits, gs, seed=2, fast=True)
+    x = np.random.default_rng(4).uniform(-1, 1, (T, K)).astype(np.float32)
+
+    def shifted(a, by):
+        d = gpu.DeviceArray(a.nbytes + 16, np.uint8)
+        raw = np.zeros(a.nbytes + 16, np.uint8)
+        raw[by:by + a.nbytes] = np.ascontiguousarray(a).view(np.uint8).reshape(-1)
+        d.upload(raw)
+        return d
+    w, s, b = shifted(fx.packed, 4), shifted(fx.s_raw, 2), shifted(fx.b_raw, 2)
+    qm = (gpu.QMat * 1)(gpu.QMat(w.ptr + 4, s.ptr + 2, b.ptr + 2, None, O))
+    dx, dy = gpu.DeviceArray.from_numpy(x), gpu.DeviceArray.zeros((T, O), np.float32)
+    gpu.check(gpu.lib.mlxr_k_qgemm(qm, K, bits, gs, 0, T, dx.ptr, K, dy.ptr, O))
+    gpu.synchronize()
+    assert np.array_equal(dy.numpy().view(np.uint32), qgemm(gpu, fx, x).view(np.uint32))
+
+
 def test_qgemm_row_scaling(gpu):
     """The prefill GEMM on rows of very different magnitude (the per-row power-of-two scaling keeps
     each row's precision), a zero row, bias, bf16 and f16 scales: every row within 1e-5 of its own
