@@ -7,24 +7,36 @@
 // and every product accumulates in fp32, so the result matches fp32 arithmetic to ~1e-5 relative.
 //
 #include "kernels.h"
+#include <algorithm>
+#include <atomic>
+#include <cmath>
+#include <type_traits>
 
 namespace mlxr {
 
 typedef __bf16 fbf16x8_t __attribute__((ext_vector_type(8)));
 typedef float ff32x4_t __attribute__((ext_vector_type(4)));
 
-// MI355X layout: a 512-thread workgroup serves one KV head (up to 4 of its query heads; G > 4 takes
-// ceil(G / 4) head groups) and two blocks of 32 queries, a light one (b) and its causal mirror
-// (nb - 1 - b): waves 0-3 take the light block's heads, waves 4-7 the heavy block's,
-// so every workgroup does the same work and the two waves on a SIMD hide each other's latency.
-// Both blocks read the same K / V tiles, copied from the paged cache straight into LDS
-// (buffer -> LDS, [key][128] bf16 with 16-byte chunks XOR-swizzled by (key & 15), two stages).
+// MI355X layout: an item is one query head's block of 32 queries; a 256-thread workgroup (a wave per SIMD,
+// two workgroups per CU, so that one's softmax runs beside the other's products) takes four items of one
+// KV head, heads fastest, over the keys its items need, or one of nsplit ranges of them: a short chunk after
+// a long context has few items, and its key ranges fill the chip instead (their partial outputs are merged
+// by flash_merge_kernel). All four items read the same K / V tiles, copied from the paged cache straight
+// into LDS (buffer -> LDS, [key][128] bf16 with 16-byte chunks XOR-swizzled by (key & 15), two stages).
 //   S^T = K Q^T   A = K rows (16-byte LDS reads), B = q * scale * log2(e) as bf16 hi + lo (registers)
-//   softmax in base 2 (exp2), per query column (two lane exchanges)
+//   softmax in base 2 (exp2), per query column (lane exchanges for the tile's max; the sums stay per lane
+//                 until the end, and the outputs are rescaled only where a max grew)
 //   O^T += V^T P^T  B = P^T from the S^T accumulators (hi + lo bf16: hardware conversions);
 //                 A = V^T read with the LDS transpose read: lane j of a 16-lane group reads key
 //                 base + (j >> 2), dims 4 (j & 3) .. + 3, and lane i receives dim i of the four
 //                 keys base .. base + 3, so V needs no transposed copy.
+// What bounds it: 128 MFMAs (the hi + lo pairs double them) and the softmax's vector work a tile and wave, the
+// two overlapped by the CU's other workgroup only in part: 3.45 us a tile for a pair, of which the MFMAs are
+// 1.7. The page number and the position go through readfirstlane, or each copy becomes a loop over lanes whose
+// buffer descriptors might differ (2048 tokens after 28000: 2990 us so, 2310 now), and whole tiles have a loop
+// of their own, without masks and without a branch around each V fragment (130 -> 126 us at 2048 after 0).
+// 1000 tokens after 7001, 40 / 8 heads: 500 us with eight items of two query blocks per workgroup in one
+// range (one workgroup per CU), 412 in this cut, 317 in four ranges.
 typedef short fp_v4s __attribute__((ext_vector_type(4)));
 typedef __bf16 fp_bf2 __attribute__((ext_vector_type(2)));
 typedef __attribute__((address_space(3))) void* fp_lptr;
@@ -40,38 +52,45 @@ __device__ __forceinline__ void split2(float x0, float x1, uint32_t& hi, uint32_
     lo = __builtin_bit_cast(uint32_t, l);
 }
 
-__global__ __launch_bounds__(512) void flash2_kernel(FlashArgs a, int nb, int ngroups) {
+struct FlashDev {
+    FlashArgs a;
+    int nb, nwg, nsplit, first;   // query blocks, workgroups per KV head and key range, key ranges, ranks dealt heaviest first
+    float* po; float* pml;        // nsplit > 1: partial outputs [split][T][nH][128], (max, sum) [split][T][nH][2]
+};
+
+__global__ __launch_bounds__(256, 2) void flash_kernel(FlashDev f) {
     extern __shared__ __attribute__((aligned(1024))) uint8_t f2_lds[];   // [2 stages][K tile, V tile]
+    const FlashArgs& a = f.a;
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int G = a.nH / a.nKV, kvh = (int)blockIdx.y / ngroups, grp = (int)blockIdx.y - kvh * ngroups;
-    const int gw = min(4, G - 4 * grp);                                  // heads of this group
-    const int hh = wave & 3, half = wave >> 2;
-    const int blight = (int)blockIdx.x, bheavy = nb - 1 - blight;
-    const int blk = half ? bheavy : blight;
-    const bool active = hh < gw && (half == 0 || bheavy != blight);
-    const int h = kvh * G + 4 * grp + min(hh, gw - 1);
-    const int pos0 = *a.dpos;
+    const int G = a.nH / a.nKV;
+    // KV heads fastest (with eight of them an XCD keeps to one), then key ranges, then item ranks: heaviest
+    // first, the ones past `first` lightest first (they share a CU with the heaviest)
+    const int per = a.nKV * f.nsplit, g = (int)blockIdx.x, rank = g / per, kvh = g % per % a.nKV, z = g % per / a.nKV;
+    const int w = rank < f.first ? f.nwg - 1 - rank : rank - f.first;
+    const int items = G * f.nb, item = 4 * w + wave, last = min(4 * w + 3, items - 1);
+    const bool active = item < items;
+    const int blk = min(item, items - 1) / G, h = kvh * G + min(item, items - 1) % G;
+    const int pos0 = __builtin_amdgcn_readfirstlane(*a.dpos);
     const int q0 = blk * 32, nq = min(32, a.T - q0);
     const int kend = pos0 + q0 + nq;                                      // this wave's keys [0, kend)
-    const int ntiles_wg = (pos0 + min(bheavy * 32 + 32, a.T) + 63) / 64;  // the heavy block's tiles
-    const int ntiles = active ? (kend + 63) / 64 : 0;
+    const int all = (pos0 + min(last / G * 32 + 32, a.T) + 63) / 64;      // the last item's tiles, of which this range's:
+    const int tile0 = all * z / f.nsplit, tile1 = all * (z + 1) / f.nsplit;
+    const int ntiles = active ? min((kend + 63) / 64, tile1) : 0;
     const int r16 = lane & 15, kq = lane >> 4;
     const float qscale = a.scale * 1.4426950408889634f;   // scores in base-2 units
 
-    // copies of tile t: wave w takes 1-KB pieces 4w .. 4w + 3 of the 32 (K: 0-15, V: 16-31)
+    // copies of tile t: wave w takes 1-KB pieces 8w .. 8w + 7 of the 32 (K: 0-15, V: 16-31)
     auto issue = [&](int t) {
-        const int page = a.pt[t];
+        const int page = __builtin_amdgcn_readfirstlane(a.pt[t]);
         uint8_t* st = f2_lds + (t & 1) * 2 * F2_TILE;
         const size_t off = ((size_t)page * a.nKV + kvh) * (size_t)F2_TILE;
-        const __amdgpu_buffer_rsrc_t kr = __builtin_amdgcn_make_buffer_rsrc((void*)((const uint8_t*)a.kc + off), 0, F2_TILE, 0x00020000);
-        const __amdgpu_buffer_rsrc_t vr = __builtin_amdgcn_make_buffer_rsrc((void*)((const uint8_t*)a.vc + off), 0, F2_TILE, 0x00020000);
+        const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc((void*)((const uint8_t*)(wave < 2 ? a.kc : a.vc) + off), 0, F2_TILE, 0x00020000);
+        st += wave < 2 ? 0 : F2_TILE;
 #pragma unroll
-        for (int i = 0; i < 4; i++) {
-            const int piece = 4 * wave + i, q = piece & 15, key = 4 * q + kq;
-            const uint32_t go = key * 256 + 16 * (r16 ^ (key & 15));
-            if (piece < 16) __builtin_amdgcn_raw_ptr_buffer_load_lds(kr, (fp_lptr)(st + q * 1024), 16, go, 0, 0, 0);
-            else __builtin_amdgcn_raw_ptr_buffer_load_lds(vr, (fp_lptr)(st + F2_TILE + q * 1024), 16, go, 0, 0, 0);
+        for (int i = 0; i < 8; i++) {
+            const int q = 8 * (wave & 1) + i, key = 4 * q + kq;
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (fp_lptr)(st + q * 1024), 16, key * 256 + 16 * (r16 ^ (key & 15)), 0, 0, 0);
         }
     };
 
@@ -101,34 +120,48 @@ __global__ __launch_bounds__(512) void flash2_kernel(FlashArgs a, int nb, int ng
         for (int qb = 0; qb < 2; qb++) o[n][qb] = ff32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
     float m[2] = {-INFINITY, -INFINITY}, l[2] = {0.0f, 0.0f};
 
-    issue(0);
-    for (int t = 0; t < ntiles_wg; t++) {
-        __builtin_amdgcn_s_waitcnt(0);       // this wave's copies of tile t landed ...
-        __builtin_amdgcn_s_barrier();        // ... and every wave's; tile t - 1's stage is free
-        if (t + 1 < ntiles_wg) issue(t + 1);
-        if (t >= ntiles) continue;
-        const uint8_t* ks = f2_lds + (t & 1) * 2 * F2_TILE;
-        const uint8_t* vs = ks + F2_TILE;
+    auto tile = [&](auto EDGEC, int t) {
+        constexpr bool EDGE = decltype(EDGEC)::value;
         const int k0 = t * 64;
+        // lane parts of the K and V addresses, opaque: their XORs are taken where used, not kept for all
+        // dims and keys across the tiles (registers that the fragments need)
+        int ln = lane;
+        asm volatile("" : "+v"(ln));
+        const uint32_t stage = (uint32_t)(t & 1) * 2 * F2_TILE, l15 = ln & 15, l4 = ln >> 4;
+        const uint32_t kaddr = stage + l15 * 256 + 16 * (l4 ^ l15);                 // ^ 64 db + 4096 kb
+        const uint32_t v15 = 4 * l4 + (l15 >> 2);                                  // key & 15 of the lane's V reads
+        const uint32_t vaddr = stage + F2_TILE + v15 * 256 + 16 * (((l15 & 3) >> 1) ^ v15) + 8 * (l15 & 1);   // ^ 32 n + 4096 (2 st + r)
 
-        // S^T tiles [kb][qb]: keys k0 + 16 kb + 4 kq + i, query 16 qb + r16
+        // S^T tiles [kb][qb]: keys k0 + 16 kb + 4 kq + i, query 16 qb + r16; the next 16 keys' fragments are
+        // read while these keys' products issue
         ff32x4_t s[4][2];
+        fbf16x8_t ka[2][4];
+        auto kread = [&](int kb) {
+#pragma unroll
+            for (int db = 0; db < 4; db++) ka[kb & 1][db] = *reinterpret_cast<const fbf16x8_t*>(f2_lds + ((kaddr ^ (64u * db)) + 4096u * kb));
+        };
+        kread(0);
 #pragma unroll
         for (int kb = 0; kb < 4; kb++) {
+            __builtin_amdgcn_sched_barrier(0);
+            if (kb < 3) kread(kb + 1);
             s[kb][0] = s[kb][1] = ff32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
-            const int key = 16 * kb + r16;
 #pragma unroll
-            for (int db = 0; db < 4; db++) {
-                const fbf16x8_t ka = *reinterpret_cast<const fbf16x8_t*>(ks + key * 256 + 16 * ((4 * db + kq) ^ (key & 15)));
+            for (int db = 0; db < 4; db++)
 #pragma unroll
-                for (int qb = 0; qb < 2; qb++) {
-                    s[kb][qb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ka, qf[db][qb][0], s[kb][qb], 0, 0, 0);
-                    s[kb][qb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ka, qf[db][qb][1], s[kb][qb], 0, 0, 0);
-                }
-            }
+                for (int p = 0; p < 2; p++)
+#pragma unroll
+                    for (int qb = 0; qb < 2; qb++) s[kb][qb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ka[kb & 1][db], qf[db][qb][p], s[kb][qb], 0, 0, 0);
         }
-        // causal mask (tiles reaching past the block's first query), base-2 online softmax
-        const bool diag = k0 + 63 > pos0 + q0;
+        __builtin_amdgcn_sched_barrier(0);
+        // V^T fragments of (step st, 16 dims n) f = 8 st + n, two ahead of the products
+        uint2 va[3][2];
+        auto vread = [&](int f) {
+#pragma unroll
+            for (int r = 0; r < 2; r++)
+                va[f % 3][r] = __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((fp_lv4)(f2_lds + ((vaddr ^ (32u * (f & 7))) + 4096u * (2 * (f >> 3) + r)))));
+        };
+        // causal mask, base-2 online softmax
         uint32_t ph[2][2][4], pl[2][2][4];   // [st][qb] P^T fragments (hi, lo), 4 dwords each
 #pragma unroll
         for (int qb = 0; qb < 2; qb++) {
@@ -138,27 +171,27 @@ __global__ __launch_bounds__(512) void flash2_kernel(FlashArgs a, int nb, int ng
             for (int kb = 0; kb < 4; kb++)
 #pragma unroll
                 for (int i = 0; i < 4; i++) {
-                    if (diag && k0 + 16 * kb + 4 * kq + i > qpos) s[kb][qb][i] = -INFINITY;
+                    if (EDGE && k0 + 16 * kb + 4 * kq + i > qpos) s[kb][qb][i] = -INFINITY;
                     mx = fmaxf(mx, s[kb][qb][i]);
                 }
             mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
             mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-            const float mn = fmaxf(m[qb], mx);
-            const float alpha = mn == -INFINITY ? 1.0f : __builtin_amdgcn_exp2f(m[qb] - mn);
-            float p[4][4], sum = 0.0f;
+            if (__any(mx > m[qb])) {
+                const float mn = fmaxf(m[qb], mx), alpha = mn == -INFINITY ? 1.0f : __builtin_amdgcn_exp2f(m[qb] - mn);
+                l[qb] *= alpha;
+                m[qb] = mn;
+#pragma unroll
+                for (int n = 0; n < 8; n++) o[n][qb] *= alpha;
+            }
+            const float ms = m[qb] == -INFINITY ? 0.0f : m[qb];   // no key yet: every p is 2^-inf
+            float p[4][4];
 #pragma unroll
             for (int kb = 0; kb < 4; kb++)
 #pragma unroll
                 for (int i = 0; i < 4; i++) {
-                    p[kb][i] = mn == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(s[kb][qb][i] - mn);
-                    sum += p[kb][i];
+                    p[kb][i] = __builtin_amdgcn_exp2f(s[kb][qb][i] - ms);
+                    l[qb] += p[kb][i];
                 }
-            sum += __shfl_xor(sum, 16, 64);
-            sum += __shfl_xor(sum, 32, 64);
-            l[qb] = l[qb] * alpha + sum;
-            m[qb] = mn;
-#pragma unroll
-            for (int n = 0; n < 8; n++) o[n][qb] *= alpha;
             // k-slots of PV step st: 0..3 = keys 16 (2 st) + 4 kq + i, 4..7 = keys 16 (2 st + 1) + 4 kq + i
 #pragma unroll
             for (int st = 0; st < 2; st++) {
@@ -168,9 +201,8 @@ __global__ __launch_bounds__(512) void flash2_kernel(FlashArgs a, int nb, int ng
                 split2(p[2 * st + 1][2], p[2 * st + 1][3], ph[st][qb][3], pl[st][qb][3]);
             }
         }
-        // keys past the chunk's last key may hold anything: zero their V (their weight is 0, and
-        // 0 * NaN is not)
-        const bool tail = k0 + 64 > kend;
+        vread(0);
+        vread(1);
 #pragma unroll
         for (int st = 0; st < 2; st++) {
             fbf16x8_t pb[2][2];
@@ -179,48 +211,145 @@ __global__ __launch_bounds__(512) void flash2_kernel(FlashArgs a, int nb, int ng
                 pb[qb][0] = __builtin_bit_cast(fbf16x8_t, uint4{ph[st][qb][0], ph[st][qb][1], ph[st][qb][2], ph[st][qb][3]});
                 pb[qb][1] = __builtin_bit_cast(fbf16x8_t, uint4{pl[st][qb][0], pl[st][qb][1], pl[st][qb][2], pl[st][qb][3]});
             }
+            // keys past the chunk's last key may hold anything: zero their V (their weight is 0, and
+            // 0 * NaN is not)
+            uint32_t vm[2][2];
+            if constexpr (EDGE) {
+#pragma unroll
+                for (int r = 0; r < 2; r++)
+#pragma unroll
+                    for (int e = 0; e < 2; e++) {
+                        const int left = kend - (k0 + 16 * (2 * st + r) + 4 * kq + 2 * e);   // keys of the pair that exist
+                        vm[r][e] = left >= 2 ? ~0u : left == 1 ? 0xFFFFu : 0u;
+                    }
+            }
 #pragma unroll
             for (int n = 0; n < 8; n++) {
-                fp_v4s vv[2];
+                const int f = 8 * st + n;
+                __builtin_amdgcn_sched_barrier(0);
+                if (f + 2 < 16) vread(f + 2);
+                if constexpr (EDGE) {
 #pragma unroll
-                for (int r = 0; r < 2; r++) {
-                    const int key = 16 * (2 * st + r) + 4 * kq + (r16 >> 2);
-                    const int c = 2 * n + ((r16 & 3) >> 1);
-                    const uint8_t* ad = vs + key * 256 + 16 * (c ^ (key & 15)) + 8 * (r16 & 1);
-                    vv[r] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((fp_lv4)(ad));
-                    if (tail) {
-#pragma unroll
-                        for (int e = 0; e < 4; e++)
-                            if (k0 + 16 * (2 * st + r) + 4 * kq + e >= kend) vv[r][e] = 0;
-                    }
+                    for (int r = 0; r < 2; r++) { va[f % 3][r].x &= vm[r][0]; va[f % 3][r].y &= vm[r][1]; }
                 }
-                const fbf16x8_t va = __builtin_bit_cast(fbf16x8_t, __builtin_shufflevector(vv[0], vv[1], 0, 1, 2, 3, 4, 5, 6, 7));
+                const fbf16x8_t v8 = __builtin_bit_cast(fbf16x8_t, uint4{va[f % 3][0].x, va[f % 3][0].y, va[f % 3][1].x, va[f % 3][1].y});
 #pragma unroll
-                for (int qb = 0; qb < 2; qb++) {
-                    o[n][qb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(va, pb[qb][0], o[n][qb], 0, 0, 0);
-                    o[n][qb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(va, pb[qb][1], o[n][qb], 0, 0, 0);
-                }
+                for (int p = 0; p < 2; p++)
+#pragma unroll
+                    for (int qb = 0; qb < 2; qb++) o[n][qb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v8, pb[qb][p], o[n][qb], 0, 0, 0);
             }
         }
-    }
+        __builtin_amdgcn_sched_barrier(0);
+    };
+
+    if (tile0 < tile1) issue(tile0);
+    auto next = [&](int t) {
+        __builtin_amdgcn_s_waitcnt(0);       // this wave's copies of tile t landed ...
+        __builtin_amdgcn_s_barrier();        // ... and every wave's; tile t - 1's stage is free
+        if (t + 1 < tile1) issue(t + 1);
+    };
+    // whole tiles: every key of theirs is at or before the block's first query
+    const int whole = max(tile0, min(ntiles, (pos0 + q0 + 1) / 64));
+    int t = tile0;
+    for (; t < whole; t++) { next(t); tile(std::false_type{}, t); }
+    for (; t < ntiles; t++) { next(t); tile(std::true_type{}, t); }
+    for (; t < tile1; t++) next(t);
     if (!active) return;
 #pragma unroll
     for (int qb = 0; qb < 2; qb++) {
+        float sum = l[qb];
+        sum += __shfl_xor(sum, 16, 64);
+        sum += __shfl_xor(sum, 32, 64);
         const int t = q0 + 16 * qb + r16;
         if (t >= a.T) continue;
-        const float inv = 1.0f / l[qb];
-        float* op = a.out + (size_t)t * a.out_stride + (size_t)h * 128 + 4 * kq;
+        const bool parts = f.nsplit > 1;
+        const size_t row = ((size_t)z * a.T + t) * a.nH + h;
+        const float inv = parts ? 1.0f : 1.0f / sum;
+        float* op = (parts ? f.po + row * 128 : a.out + (size_t)t * a.out_stride + (size_t)h * 128) + 4 * kq;
+        if (parts && kq == 0) *reinterpret_cast<float2*>(f.pml + 2 * row) = float2{m[qb], sum};
 #pragma unroll
         for (int n = 0; n < 8; n++)
             *reinterpret_cast<float4*>(op + 16 * n) = float4{o[n][qb][0] * inv, o[n][qb][1] * inv, o[n][qb][2] * inv, o[n][qb][3] * inv};
     }
 }
 
+// One wave per (token, head): the key ranges' partial outputs, weighted by 2^(max - largest max), in order.
+__global__ __launch_bounds__(256) void flash_merge_kernel(FlashDev f) {
+    const FlashArgs& a = f.a;
+    const int lane = threadIdx.x & 63, i = (int)blockIdx.x * 4 + (threadIdx.x >> 6), n = a.T * a.nH;
+    if (i >= n) return;
+    const float2 ml = lane < f.nsplit ? *reinterpret_cast<const float2*>(f.pml + 2 * ((size_t)lane * n + i)) : float2{-INFINITY, 0.0f};
+    const float M = wave_max(ml.x), wt = ml.x == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(ml.x - M);
+    const float inv = 1.0f / wave_sum(wt * ml.y);
+    float2 o = {0.0f, 0.0f};
+    for (int z = 0; z < f.nsplit; z += 8) {
+        float2 v[8];
+#pragma unroll
+        for (int j = 0; j < 8; j++) v[j] = *reinterpret_cast<const float2*>(f.po + ((size_t)min(z + j, f.nsplit - 1) * n + i) * 128 + 2 * lane);
+#pragma unroll
+        for (int j = 0; j < 8; j++)
+            if (z + j < f.nsplit) {
+                const float wz = __shfl(wt, z + j, 64);
+                o.x += v[j].x * wz; o.y += v[j].y * wz;
+            }
+    }
+    float* op = a.out + (size_t)(i / a.nH) * a.out_stride + (size_t)(i % a.nH) * 128 + 2 * lane;
+    op[0] = o.x * inv; op[1] = o.y * inv;
+}
+
+static int flash_workgroups(const FlashArgs& a) { return (a.nH / a.nKV * ((a.T + 31) / 32) + 3) / 4 * a.nKV; }
+static int flash_cus() {
+    static std::atomic<int> cus{0};
+    if (int c = cus.load(std::memory_order_relaxed)) return c;
+    int dev = 0, n = 0;
+    if (hipGetDevice(&dev) == hipSuccess && hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && n > 0) cus = n;
+    return n > 0 ? n : 256;
+}
+// Key ranges by expected time. A workgroup alone on its CU takes 1.95 us a tile, two of them 3.45 us a tile
+// each (so pairs gain 1.13x, and a launch of fewer than a workgroup per CU gains the whole cut); the merge
+// reads and writes the partial outputs at ~3 TB/s behind a launch of ~5 us. The model is within 15% of the
+// times measured for 1 .. 32 ranges on 18 shapes (16 .. 2048 tokens after 0 .. 28000, 2 .. 40 heads), of
+// which it takes ranges for all but the first chunks with a workgroup per CU or more: 2048 tokens at 0, 32
+// heads, are 78 us in one range and 98 in two; 16 tokens after 7000, 40 heads, are 216 and 19 in sixteen.
+static int flash_splits(const FlashArgs& a, size_t part_floats) {
+    constexpr float ALONE = 1.95f, PAIR = 3.45f;
+    const int cus = flash_cus(), wgs = flash_workgroups(a);
+    const float tmax = float((a.pos + a.T + 63) / 64), tmin = float((a.pos + std::min(a.T, 32) + 63) / 64), avg = 0.5f * (tmin + tmax);
+    int best = 1;
+    float bestus = 0.0f;
+    for (int ns = 1; ns <= 32 && 2 * ns <= std::max(2.0f, tmax); ns++) {
+        if (ns > 1 && (size_t)ns * a.T * a.nH * 130 > part_floats) break;
+        const float n = (float)wgs * ns;
+        float us;
+        if (n <= cus) us = ceilf(tmax / ns) * ALONE;
+        else if (n <= 2 * cus) us = (tmin * PAIR + (tmax - tmin) * ALONE) / ns;   // heaviest beside lightest
+        else {
+            const float rounds = floorf(n / (2 * cus)), rest = n - rounds * 2 * cus;
+            us = (rounds * PAIR + (rest == 0 ? 0.0f : rest <= cus ? ALONE : PAIR)) * avg / ns;
+        }
+        if (ns > 1) us += 5.0f + (float)a.T * a.nH * ns * (2 * 520 / 3e6f);
+        if (ns == 1 || us < bestus) { best = ns; bestus = us; }
+    }
+    return best;
+}
+size_t flash_part_floats(const FlashArgs& a) {
+    const int ns = flash_splits(a, FLASH_PART_FLOATS);
+    return ns > 1 ? (size_t)ns * a.T * a.nH * 130 : 0;
+}
+
 hipError_t launch_flash_prefill(const FlashArgs& a, hipStream_t s) {
     if (a.D != 128 || a.nKV < 1 || a.nH % a.nKV || a.nH / a.nKV > 8 || a.T < 1) return hipErrorInvalidValue;
-    const int G = a.nH / a.nKV, ngroups = (G + 3) / 4;
-    const int nb = (a.T + 31) / 32, npair = (nb + 1) / 2;
-    hipLaunchKernelGGL(flash2_kernel, dim3(npair, a.nKV * ngroups), dim3(512), 4 * F2_TILE, s, a, nb, ngroups);
+    const int cus = flash_cus();
+    FlashDev f{};
+    f.a = a;
+    f.nb = (a.T + 31) / 32;
+    f.nwg = flash_workgroups(a) / a.nKV;
+    f.nsplit = flash_splits(a, a.part ? a.part_floats : 0);
+    const int total = f.nwg * a.nKV * f.nsplit;
+    f.first = total > cus && total <= 2 * cus ? cus / (a.nKV * f.nsplit) : f.nwg;
+    if (f.nsplit > 1) { f.po = a.part; f.pml = a.part + (size_t)f.nsplit * a.T * a.nH * 128; }
+    hipLaunchKernelGGL(flash_kernel, dim3(total), dim3(256), 4 * F2_TILE, s, f);
+    if (f.nsplit > 1) hipLaunchKernelGGL(flash_merge_kernel, dim3((a.T * a.nH + 3) / 4), dim3(256), 0, s, f);
     return hipGetLastError();
 }
 

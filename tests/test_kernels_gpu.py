@@ -677,6 +677,31 @@ def test_flash_prefill(gpu, nH, nKV, offset, T):
         assert max_rel_err(got[t], ref) < 1e-4, (t, max_rel_err(got[t], ref))
 
 
+@pytest.mark.parametrize("nH,nKV,offset,T", [(2, 2, 3000, 33), (5, 1, 2040, 16), (16, 2, 4095, 9), (6, 2, 1999, 77), (40, 8, 900, 40)])
+def test_flash_key_ranges(gpu, nH, nKV, offset, T):
+    """Short chunks after a long context, whose keys the launch cuts into ranges merged afterwards: item
+    counts that are no multiple of four (3 heads x 3 blocks, 5 x 1, 1 x 2), ranges that end before a
+    block's last key or hold none of its keys, a last tile of one key and of 64, NaN past the last key.
+    A few tokens against the reference attention, 1e-4 relative (q and p as hi + lo bf16 pairs, ~2^-16,
+    fp32 sums; the merge adds at most 32 fp32 terms). One token's query is a multiple of one key, whose
+    range then outweighs the others."""
+    D, S = 128, (offset + T + 127) // 64 * 64
+    rng = np.random.default_rng(nH + T)
+    kc = bf16_to_f32(bf16_round(rng.uniform(-1, 1, (nKV, S, D)).astype(np.float32)))
+    vc = bf16_to_f32(bf16_round(rng.uniform(-1, 1, (nKV, S, D)).astype(np.float32)))
+    kc[:, offset + T:] = np.nan
+    vc[:, offset + T:] = np.nan
+    q = rng.uniform(-1, 1, (T, nH, D)).astype(np.float32)
+    q[T // 2] = 3 * kc[0, offset // 3]      # one token whose softmax is nearly one key's
+    scale = 3 / np.sqrt(D)
+    got = run_flash(gpu, q, kc, vc, nH, nKV, offset, T, scale)
+    assert np.all(np.isfinite(got))
+    kref, vref = np.nan_to_num(kc), np.nan_to_num(vc)
+    for t in sorted({0, 1, T // 2, T - 2, T - 1}):
+        ref = oracle.attention(q[t], kref, vref, nH, nKV, offset + t, scale)
+        assert max_rel_err(got[t], ref) < 1e-4, (t, max_rel_err(got[t], ref))
+
+
 @pytest.mark.parametrize("nH,nKV", [(4, 2), (8, 2), (10, 2)])
 def test_attention_over_lists(gpu, nH, nKV):
     """attentionOverTheList (SparseAttentionTests.swift:214-297): the full list is bit-identical to
