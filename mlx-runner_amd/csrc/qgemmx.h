@@ -475,6 +475,7 @@ __device__ __forceinline__ void qgemmx_body(const QGemmXDev& a, uint8_t* lds, in
         }
     }
     if (a.S > 1) {
+        __builtin_amdgcn_s_waitcnt(0);   // the partial tile is stored (and visible at agent scope) before its counter moves
         __syncthreads();
         __shared__ int last;
         if (tid == 0) last = __hip_atomic_fetch_add(a.cnt + tile, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) == (unsigned)(a.S - 1);
