@@ -66,6 +66,12 @@ template <typename T> int ensure_buf(T*& p, size_t& have, size_t need) {
     have = need;
     return MLXR_OK;
 }
+int ensure_qsplit() {
+    if (g_qsplit) return MLXR_OK;
+    if (int rc = ensure_buf(g_qsplit, g_qsplit_floats, QGEMM_SPLIT_FLOATS)) return rc;
+    CK(hipMemset(g_qsplit, 0, QGEMM_SPLIT_FLOATS * 4));
+    return MLXR_OK;
+}
 bool bits_ok(int b) { return b == 2 || b == 3 || b == 4 || b == 5 || b == 6 || b == 8; }
 int check_quant(int K, int bits, int gs, int st) {
     if (!bits_ok(bits)) return set_error(MLXR_E_UNSUPPORTED, "bits must be 2, 3, 4, 5, 6 or 8");
@@ -244,14 +250,8 @@ int mlxr_k_qmm(const mlxr_qmat* parts, int nparts, int K, int bits, int gs, int 
     QmmSmallArgs a; a.nparts = nparts;
     for (int i = 0; i < nparts; i++) a.part[i] = qmat(parts[i]);
     a.K = K; a.bits = bits; a.gs = gs; a.st = st; a.O = O; a.T = T; a.x = x; a.x_stride = x_stride; a.y = y; a.y_stride = y_stride;
-    if (qmmx_supported(K, bits, gs)) {
-        if (int rc = ensure_buf(g_xbf, g_xbf_elems, (size_t)T * K)) return rc;
-        if (int rc = ensure_buf(g_xlo, g_xlo_elems, (size_t)T * K)) return rc;
-        if (int rc = ensure_buf(g_xgs, g_xgs_elems, qgemm_gsum_floats(T, K, gs))) return rc;
-        if (int rc = ensure_buf(g_xsc, g_xsc_elems, (size_t)T)) return rc;
-        if (int rc = ensure_buf(g_xnz, g_xnz_elems, (size_t)T)) return rc;
-        a.xbf = g_xbf; a.xlo = g_xlo; a.xgs = g_xgs; a.xsc = g_xsc; a.xnz = g_xnz;
-    }
+    if (ensure_qsplit() != MLXR_OK) (void)hipGetLastError();   // no room: no K ranges
+    a.split = g_qsplit; a.split_floats = g_qsplit_floats;
     return done(launch_qmm_small(a, g_stream));
 }
 
@@ -267,10 +267,7 @@ int mlxr_k_qgemm(const mlxr_qmat* mat, int K, int bits, int gs, int st, int T, c
     if (int rc = ensure_buf(g_xgs, g_xgs_elems, qgemm_gsum_floats(T, K, gs))) return rc;
     if (int rc = ensure_buf(g_wsb, g_wsb_elems, qgemm_scale_halves(mat->O, K, gs))) return rc;
     if (int rc = ensure_buf(g_xnz, g_xnz_elems, (size_t)T)) return rc;
-    if (!g_qsplit) {
-        if (int rc = ensure_buf(g_qsplit, g_qsplit_floats, QGEMM_SPLIT_FLOATS)) return rc;
-        CK(hipMemset(g_qsplit, 0, QGEMM_SPLIT_FLOATS * 4));
-    }
+    if (int rc = ensure_qsplit()) return rc;
     QGemmArgs a; a.m = qmat(*mat); a.K = K; a.bits = bits; a.gs = gs; a.st = st; a.O = mat->O; a.T = T;
     a.x = x; a.x_stride = x_stride; a.y = y; a.y_stride = y_stride; a.xbf = g_xbf; a.xsc = g_xsc;
     a.xlo = g_xlo; a.xgs = g_xgs; a.xnz = g_xnz; a.wsb = g_wsb;

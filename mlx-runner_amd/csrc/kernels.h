@@ -38,14 +38,11 @@ struct QmmSmallArgs {
     int K = 0, bits = 4, gs = 64, st = 0, O = 0, T = 1;
     const float* x = nullptr; int x_stride = 0;
     float* y = nullptr; int y_stride = 0;
-    // optional pre-pass scratch (as QGemmArgs'): with it, the shapes qmmx_supported accepts (widths
-    // 2 / 3 / 4 / 6 / 8) run on the matrix cores (launch_qmmx); without it, or for other shapes, on
-    // the fp32 vector path
-    uint16_t* xbf = nullptr; uint16_t* xlo = nullptr; float* xgs = nullptr; float* xsc = nullptr; int* xnz = nullptr;
+    float* split = nullptr; size_t split_floats = 0;   // optional scratch for K ranges, as QGemmArgs' (the same buffer serves both)
 };
 hipError_t launch_qmm_small(const QmmSmallArgs& a, hipStream_t s);
-bool qmmx_supported(int K, int bits, int gs);
-hipError_t launch_qmmx(const QmmSmallArgs& a, hipStream_t s);
+bool qmb_supported(int gs);                             // group sizes of the matrix-core kernel; others run on the fp32 vector path
+hipError_t launch_qmb(const QmmSmallArgs& a, hipStream_t s);
 
 // Prefill GEMM over the MLX layout, any code width: Y[T][O] = X[T][K] W[O][K]^T (+bias) with exact
 // codes on the f16 matrix cores, x as f16 hi + lo (per-row power-of-two scale) and the group scale

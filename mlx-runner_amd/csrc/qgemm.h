@@ -1,4 +1,4 @@
-// Shared by the MLX-layout GEMM (qgemmx.h) and the small batch (gemm.hip): operand types and constants.
+// Shared by the MLX-layout GEMM (qgemmx.h, gemm.hip) and the small batch (qmm.hip): operand types and constants.
 #pragma once
 #include "kernels.h"
 

@@ -132,6 +132,43 @@ def test_qmm_small_batch_wide_loads(gpu, bits, gs, st):
             assert max_rel_err(dy.numpy(), ref) < TOL, (T, bf16_x)
 
 
+@pytest.mark.parametrize("gs", [32, 64, 128])
+@pytest.mark.parametrize("bits", [2, 3, 4, 5, 6, 8])
+def test_qmm_small_batch_cuts(gpu, bits, gs):
+    """The small-batch kernel's cuts around their edges: last chunks of 64 (gs 128: 128) codes, K ranges of
+    uneven length met in the scratch (8320 inputs, 70 rows in three parts with bias), ranges of several
+    slices (8320 inputs, 8200 rows), two or four tiles per wave (20000 rows), one row; a token's
+    magnitude changing by 2^40 along K and from token to token, padded strides. The bound is the arithmetic's: fp32
+    sums of K / 32 products of 32 terms and of at most 16 ranges, x = hi + lo to 2^-21 of its slice's largest."""
+    rng = np.random.default_rng(bits * 100 + gs)
+    tail = 128 if gs == 128 else 64
+    for K, Os, T in ((8192 + 128, (33, 20, 17), 8), (8192 + 128, (8200,), 3), (256 + tail, (20000,), 5), (1024 + 128, (1,), 2), (tail, (65,), 7)):
+        fxs = [QuantFixture(O, K, bits, gs, st="f16" if bits % 2 else "bf16", seed=O + K, with_bias=len(Os) > 1, fast=True) for O in Os]
+        O, xs = sum(Os), K + 8
+        qm = (gpu.QMat * len(fxs))(*[f.device(gpu) for f in fxs])
+        x = rng.normal(0, 1, (T, K)) * 10.0 ** rng.integers(-3, 4, (T, 1))
+        if T > 2:
+            x[1] *= 2.0 ** np.linspace(-20, 20, K)
+        xp = np.full((T, xs), np.nan, np.float32)
+        xp[:, :K] = x
+        dx, dy = gpu.DeviceArray.from_numpy(xp), gpu.DeviceArray.from_numpy(np.full((T, O + 3), np.nan, np.float32))
+        for _ in range(2):      # the scratch's counters are back at zero
+            gpu.check(gpu.lib.mlxr_k_qmm(qm, len(fxs), K, bits, gs, bits % 2, T, dx.ptr, xs, dy.ptr, O + 3))
+            gpu.synchronize()
+            got, col = dy.numpy(), 0
+            assert np.all(np.isnan(got[:, O:]))
+            xf, top = xp[:, :K].astype(np.float64), np.abs(xp[:, :K])
+            big = np.concatenate([np.broadcast_to(top[:, i:i + 1024].max(1, keepdims=True), top[:, i:i + 1024].shape) for i in range(0, K, 1024)], axis=1)
+            for f in fxs:
+                g = np.repeat(np.arange(K // gs), gs)
+                sc, bi = f.scales[:, g].astype(np.float64), f.biases[:, g].astype(np.float64)
+                ref = xf @ (f.codes * sc + bi).T + (f.bias.astype(np.float64) if f.bias is not None else 0.0)
+                size = (f.codes * np.abs(sc) + np.abs(bi)).T
+                tol = (K / 32 + 64) * 2.0**-24 * (top @ size) + 2.0**-21 * 2.0**-11 * (big @ size) + 1e-6
+                assert np.all(np.abs(got[:, col:col + f.O] - ref) <= tol), (K, Os, T)
+                col += f.O
+
+
 def qgemm(mlxr, fx, x):
     T = x.shape[0]
     qm = (mlxr.QMat * 1)(fx.device(mlxr))
