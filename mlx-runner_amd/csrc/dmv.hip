@@ -192,13 +192,14 @@ __global__ void __launch_bounds__(MK_THREADS) dpack_mv_split_kernel(MvPhaseDesc 
     q.tstride = NF;
     q.bias[0] = q.bias[1] = q.bias[2] = nullptr;
     dmv_body<FB, DMV_OUT_PARTIAL, true>(q, x + fa * FB * 128, nullptr, 0.0f, part + (size_t)sl * p.rows, tpw, w, nw);
-    // the partial rows are stored (and visible at agent scope) before the tiles' counters move
+    // the partial rows are stored through to memory (agent scope) and waited for before the tiles' counters
+    // move, so the hand-over needs no write-back or invalidation of the caches (an acquire-release's)
     __builtin_amdgcn_s_waitcnt(0);
     __syncthreads();
     __shared__ int last[MK_TPW];
     const MvGeom<FB> g = mv_geom<FB>(q, w, nw, 0);
     if ((int)threadIdx.x < g.nt)
-        last[threadIdx.x] = __hip_atomic_fetch_add(cnt + g.t0 + threadIdx.x, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) == (unsigned)(S - 1);
+        last[threadIdx.x] = __hip_atomic_fetch_add(cnt + g.t0 + threadIdx.x, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == (unsigned)(S - 1);
     __syncthreads();
     for (int i = threadIdx.x; i < g.nt * 16; i += MK_THREADS) {
         if (!last[i >> 4]) continue;
@@ -511,13 +512,14 @@ __global__ void __launch_bounds__(MK_THREADS) dpack_mm_kernel(MmArgs a) {
         else put(tl, row, tk, v * unscale[tk]);
     }
     if (direct) return;
-    // the slices' partials are stored (and visible at agent scope) before the tiles' counters move;
+    // the slices' partials are stored through to memory (agent scope) and waited for before the tiles' counters
+    // move (no write-back or invalidation of the caches, as an acquire-release would do);
     // the tile's last workgroup sums them in slice order
     __builtin_amdgcn_s_waitcnt(0);
     __syncthreads();
     int* last = reinterpret_cast<int*>(slots);
     if ((int)threadIdx.x < g0.nt)
-        last[threadIdx.x] = __hip_atomic_fetch_add(a.cnt + T0 + threadIdx.x, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) == (unsigned)(S - 1);
+        last[threadIdx.x] = __hip_atomic_fetch_add(a.cnt + T0 + threadIdx.x, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == (unsigned)(S - 1);
     __syncthreads();
     auto partial = [&](int tl, int row, int tk) {
         float v = 0.0f;

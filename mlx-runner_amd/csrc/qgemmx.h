@@ -475,10 +475,12 @@ __device__ __forceinline__ void qgemmx_body(const QGemmXDev& a, uint8_t* lds, in
         }
     }
     if (a.S > 1) {
-        __builtin_amdgcn_s_waitcnt(0);   // the partial tile is stored (and visible at agent scope) before its counter moves
+        // the partial tile is stored through to memory (agent scope) and waited for before its counter moves: no
+        // write-back or invalidation of the caches (an acquire-release's)
+        __builtin_amdgcn_s_waitcnt(0);
         __syncthreads();
         __shared__ int last;
-        if (tid == 0) last = __hip_atomic_fetch_add(a.cnt + tile, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) == (unsigned)(a.S - 1);
+        if (tid == 0) last = __hip_atomic_fetch_add(a.cnt + tile, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == (unsigned)(a.S - 1);
         __syncthreads();
         if (!last) return;
         if (tid == 0) __hip_atomic_store(a.cnt + tile, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
