@@ -90,8 +90,9 @@ __device__ __forceinline__ float silu_mul(float g, float u) { return (g / (1.0f 
 
 // XNORM: x is normalised into LDS by the workgroup (K floats). XCOPY: x is copied into LDS as it is
 // (the four waves then read it from there: each wave's x would otherwise come through L2 once per
-// four rows, more bytes than its weights). KS: the waves split K over the same rows.
-template <int BITS, int ST, bool XNORM, bool KS, bool XCOPY = false>
+// four rows, more bytes than its weights). KS: the waves split K over the same rows; 2: a lane's next two
+// chunks are requested together, before the arithmetic of the first.
+template <int BITS, int ST, bool XNORM, int KS, bool XCOPY = false>
 __global__ __launch_bounds__(256) void qmv_kernel(QmvDev a) {
     constexpr int R = KS ? QMV_KS_ROWS : QMV_ROWS;   // rows per wave (split K: per workgroup)
     extern __shared__ __attribute__((aligned(16))) float xs_lds[];
@@ -160,26 +161,41 @@ __global__ __launch_bounds__(256) void qmv_kernel(QmvDev a) {
     for (int r = 0; r < R; r++) acc[r] = 0.0f;
     const int nchunks = K >> 5;
     const int cq0 = KS ? nchunks * wave / QMV_WAVES : 0, cq1 = KS ? nchunks * (wave + 1) / QMV_WAVES : nchunks;
-    for (int c = cq0 + lane; c < cq1; c += 64) {
-        const int k0 = c << 5;
-        uint32_t w[R][BITS];
-#pragma unroll
-        for (int r = 0; r < R; r++) load_chunk<BITS>(wp[r] + (int64_t)c * (4 * BITS), w[r]);
+    auto chunk = [&](int c, const uint32_t (&w)[R][BITS], const uint16_t (&s)[R], const uint16_t (&b)[R]) {
         float x[32];
 #pragma unroll
         for (int i = 0; i < 8; i++) {
-            const float4 v = *reinterpret_cast<const float4*>(xsrc + k0 + 4 * i);
+            const float4 v = *reinterpret_cast<const float4*>(xsrc + (c << 5) + 4 * i);
             x[4 * i] = v.x; x[4 * i + 1] = v.y; x[4 * i + 2] = v.z; x[4 * i + 3] = v.w;
         }
         float xsum = 0.0f;
 #pragma unroll
         for (int j = 0; j < 32; j++) xsum += x[j];
-        const int g = k0 / a.gs;
 #pragma unroll
-        for (int r = 0; r < R; r++) {
-            const float s = ld_scale<ST>(sp[r] + g), b = ld_scale<ST>(bp[r] + g);
-            const float d = chunk_dot<BITS>(w[r], x);
-            acc[r] += s * d + b * xsum;
+        for (int r = 0; r < R; r++) acc[r] += ld_scale<ST>(&s[r]) * chunk_dot<BITS>(w[r], x) + ld_scale<ST>(&b[r]) * xsum;
+    };
+    auto fetch = [&](int c, uint32_t (&w)[R][BITS], uint16_t (&s)[R], uint16_t (&b)[R]) {
+        const int g = (c << 5) / a.gs;
+#pragma unroll
+        for (int r = 0; r < R; r++) { load_chunk<BITS>(wp[r] + (int64_t)c * (4 * BITS), w[r]); s[r] = sp[r][g]; b[r] = bp[r][g]; }
+    };
+    if constexpr (KS == 2) {
+        uint32_t w0[R][BITS], w1[R][BITS];
+        uint16_t s0[R], b0[R], s1[R], b1[R];
+        for (int c = cq0 + lane; c < cq1; c += 128) {
+            fetch(c, w0, s0, b0);
+            const bool two = c + 64 < cq1;
+            if (two) fetch(c + 64, w1, s1, b1);
+            __builtin_amdgcn_sched_barrier(0);
+            chunk(c, w0, s0, b0);
+            if (two) chunk(c + 64, w1, s1, b1);
+        }
+    } else {
+        for (int c = cq0 + lane; c < cq1; c += 64) {
+            uint32_t w[R][BITS];
+            uint16_t s[R], b[R];
+            fetch(c, w, s, b);
+            chunk(c, w, s, b);
         }
     }
 #pragma unroll
@@ -224,7 +240,7 @@ __global__ __launch_bounds__(256) void qmv_kernel(QmvDev a) {
 }
 
 template <int BITS, int ST, bool XNORM>
-static hipError_t qmv_launch(const QmvDev& d, bool ks, int grid, size_t lds, hipStream_t s) {
+static hipError_t qmv_launch(const QmvDev& d, int ks, int grid, size_t lds, hipStream_t s) {
     // x staged in LDS where it fits the default 64 KiB (XNORM stages it anyway), not when the waves
     // split K (each reads a quarter of it), and at 8 bits only over many rounds of workgroups
     // (measured on the sweep cells: 4096 -> 14336 rows 13.0 -> 10.9 us at 4 bits but 20.2 -> 22.1 at 8
@@ -232,18 +248,15 @@ static hipError_t qmv_launch(const QmvDev& d, bool ks, int grid, size_t lds, hip
     // 13-19 -> 15-21 us)
     const bool xc = !XNORM && !ks && (size_t)d.K * sizeof(float) <= 65536 && (BITS < 8 || grid >= 2048);
     if (xc) lds = (size_t)d.K * sizeof(float);
-    if (ks) {
-        if (xc) hipLaunchKernelGGL((qmv_kernel<BITS, ST, XNORM, true, true>), dim3(grid), dim3(256), lds, s, d);
-        else hipLaunchKernelGGL((qmv_kernel<BITS, ST, XNORM, true>), dim3(grid), dim3(256), lds, s, d);
-    } else {
-        if (xc) hipLaunchKernelGGL((qmv_kernel<BITS, ST, XNORM, false, true>), dim3(grid), dim3(256), lds, s, d);
-        else hipLaunchKernelGGL((qmv_kernel<BITS, ST, XNORM, false>), dim3(grid), dim3(256), lds, s, d);
-    }
+    if (ks == 2) hipLaunchKernelGGL((qmv_kernel<BITS, ST, XNORM, 2>), dim3(grid), dim3(256), lds, s, d);
+    else if (ks) hipLaunchKernelGGL((qmv_kernel<BITS, ST, XNORM, 1>), dim3(grid), dim3(256), lds, s, d);
+    else if (xc) hipLaunchKernelGGL((qmv_kernel<BITS, ST, XNORM, 0, true>), dim3(grid), dim3(256), lds, s, d);
+    else hipLaunchKernelGGL((qmv_kernel<BITS, ST, XNORM, 0>), dim3(grid), dim3(256), lds, s, d);
     return hipGetLastError();
 }
 
 template <int BITS>
-static hipError_t qmv_dispatch_st(const QmvDev& d, int st, bool xn, bool ks, int grid, size_t lds, hipStream_t s) {
+static hipError_t qmv_dispatch_st(const QmvDev& d, int st, bool xn, int ks, int grid, size_t lds, hipStream_t s) {
     if (st == 0) return xn ? qmv_launch<BITS, 0, true>(d, ks, grid, lds, s) : qmv_launch<BITS, 0, false>(d, ks, grid, lds, s);
     return xn ? qmv_launch<BITS, 1, true>(d, ks, grid, lds, s) : qmv_launch<BITS, 1, false>(d, ks, grid, lds, s);
 }
@@ -259,10 +272,19 @@ hipError_t launch_qmv(const QmvArgs& a, hipStream_t s) {
     d.x = a.x; d.norm_w = a.norm_w; d.eps = a.eps; d.y = a.y;
     // measured on the 14336-input sweep cells: 3 / 4 / 6 bits 19.3 / 18.9 / 21.1 -> 12.9 / 13.5 / 15.6 us;
     // 8-bit rows (twice the bytes per chunk, each wave's loads already busy) 18.6 -> 21.9, so not those
-    const bool ks = (a.K >> 5) >= 64 * QMV_WAVES && a.bits < 8;
-    const int rows = ks ? QMV_KS_ROWS : QMV_ROWS;
-    const int per_wg = (ks ? 1 : QMV_WAVES) * (a.epi == EPI_GATED ? rows / 2 : rows);
+    const bool split = (a.K >> 5) >= 64 * QMV_WAVES && a.bits < 8;
+    const int rows = split ? QMV_KS_ROWS : QMV_ROWS;
+    const int per_wg = (split ? 1 : QMV_WAVES) * (a.epi == EPI_GATED ? rows / 2 : rows);
     const int grid = (a.O + per_wg - 1) / per_wg;
+    // Such a wave has one to a few chunks a lane, and each was a round trip to memory of its own. Two chunks
+    // in flight cost registers (6 bits: 228, two workgroups per CU), which tells where many rounds of
+    // workgroups hide the round trips: so where the launch is short, or the waves have two chunks of wide
+    // codes, or more than two of any. us per launch, one -> two chunks: 14336 -> 4096 at 3 / 4 / 6 bits 14.2 ->
+    // 13.9, 15.9 -> 15.1, 19.3 -> 17.6; 14336 -> 8192 6 bits 30.2 -> 28.0; 14336 -> 28672 6 bits 111 -> 82;
+    // 27648 -> 16384 5 bits 122 -> 90; 27648 -> 32768 2 bits 130 -> 108; but 14336 -> 12288 3 bits 32.6 -> 33.8,
+    // 14336 -> 28672 4 bits 66.0 -> 66.4 and 8192 -> 28672 6 bits 43.7 -> 49.6.
+    const bool two = grid <= 1024 || (a.bits >= 5 && a.K > 8192) || a.K > 16384;
+    const int ks = !split ? 0 : two ? 2 : 1;
     const bool xn = a.norm_w != nullptr;
     const size_t lds = xn ? (size_t)a.K * sizeof(float) : 0;
     switch (a.bits) {

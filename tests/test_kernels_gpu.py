@@ -58,6 +58,35 @@ def test_qmv_partial_passes(gpu, K):
         assert max_rel_err(qmv(gpu, [fx], x), fx.oracle(oracle).matmul_f64(x)[0]) < TOL
 
 
+@pytest.mark.parametrize("bits,K,gs,O", [(4, 8192, 64, 20), (3, 8256, 32, 9), (6, 14336, 128, 33), (2, 16448, 32, 8), (5, 25600, 64, 17),
+                                         (4, 8256, 32, 8201), (5, 8192, 64, 8193), (6, 8256, 32, 8195)])
+def test_qmv_split_k(gpu, bits, K, gs, O):
+    """Rows whose K is split over a workgroup's waves, one or two chunks of 32 codes in flight per lane: one
+    chunk a lane, a ragged second, a third, rows that end inside a workgroup of eight, and launches past
+    1024 workgroups (one chunk in flight, or two for wide codes over more than one chunk). The bound is the
+    arithmetic's, elementwise: a product passes through at most 64 fp32 roundings (32 in its chunk, the group's
+    scale and bias, the lane's chunks, the tree over lanes, the waves), each 2^-24 of the row's sum of |terms|.
+    The accumulate, fused norm and gated epilogues on the small launches."""
+    fx = QuantFixture(O, K, bits, gs, seed=K + bits, fast=True)
+    rng = np.random.default_rng(K + O)
+    x = rng.normal(0, 1, K).astype(np.float32)
+    ref = fx.oracle(oracle).matmul_f64(x)[0].astype(np.float64)
+    sums = np.abs(x).reshape(-1, gs)
+    size = np.einsum("ogk,gk->og", fx.codes.astype(np.float32).reshape(O, -1, gs), sums) * fx.scales + np.abs(fx.biases) * sums.sum(1)
+    tol = 64 * 2.0**-24 * size.sum(1)
+    assert np.all(np.abs(qmv(gpu, [fx], x) - ref) <= tol)
+    if O > 64 or K > 14336:
+        return
+    y0 = rng.normal(0, 1, O).astype(np.float32)
+    assert np.all(np.abs(qmv(gpu, [fx], x, epi=1, y0=y0) - (y0 + ref)) <= tol + 1e-6)
+    w = rng.uniform(0.5, 1.5, K).astype(np.float32)
+    up = QuantFixture(O, K, bits, gs, seed=K + bits + 1, fast=True)
+    xn = oracle.rms_norm(x[None], w, 1e-6)[0]
+    g, u = (f.oracle(oracle).matmul_f64(xn)[0] for f in (fx, up))
+    gated = np.array([oracle.lib.orc_silu_mul(float(a), float(b)) for a, b in zip(g, u)], np.float32)
+    assert max_rel_err(qmv(gpu, [fx, up], x, norm_w=w, epi=2), gated) < TOL
+
+
 def test_fused_qkv_with_bias_matches_separate(gpu):
     """fusedDecodeWithBiasMatchesSeparate (KernelTests.swift:214-227)."""
     K = 256
