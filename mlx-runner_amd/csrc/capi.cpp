@@ -449,9 +449,6 @@ int mlxr_k_flash_prefill(const float* q, int q_stride, const void* kcache, const
         if (int rc = set_pos(offset)) return rc;
         FlashArgs a; a.q = q; a.q_stride = q_stride; a.kc = (const uint16_t*)kcache; a.vc = (const uint16_t*)vcache; a.pt = g_pt;
         a.out = out; a.out_stride = out_stride; a.D = D; a.nH = nH; a.nKV = nKV; a.T = T; a.dpos = g_pos; a.scale = scale;
-        a.pos = offset;
-        if (ensure_buf(g_part, g_part_floats, flash_part_floats(a)) != MLXR_OK) (void)hipGetLastError();   // no room: no key ranges
-        a.part = g_part; a.part_floats = g_part_floats;
         return done(launch_flash_prefill(a, g_stream));
     }
 }

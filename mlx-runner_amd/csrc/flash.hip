@@ -7,9 +7,7 @@
 // and every product accumulates in fp32, so the result matches fp32 arithmetic to ~1e-5 relative.
 //
 #include "kernels.h"
-#include <algorithm>
 #include <atomic>
-#include <cmath>
 #include <type_traits>
 
 namespace mlxr {
@@ -19,13 +17,15 @@ typedef float ff32x4_t __attribute__((ext_vector_type(4)));
 
 // MI355X layout: an item is one query head's block of 32 queries; a 256-thread workgroup (a wave per SIMD,
 // two workgroups per CU, so that one's softmax runs beside the other's products) takes four items of one
-// KV head, heads fastest, over the keys its items need, or one of nsplit ranges of them: a short chunk after
-// a long context has few items, and its key ranges fill the chip instead (their partial outputs are merged
-// by flash_merge_kernel). All four items read the same K / V tiles, copied from the paged cache straight
+// KV head, heads fastest. All four items read the same K / V tiles, copied from the paged cache straight
 // into LDS (buffer -> LDS, [key][128] bf16 with 16-byte chunks XOR-swizzled by (key & 15), two stages).
+// A query walks every key tile from position 0 in order, whatever the chunk or its place in it (tiles past
+// its last key change nothing), so its output has the same bits however a prompt is cut into chunks. Key
+// ranges on workgroups of their own, as many as leave no CU idle, did not keep that (16 tokens after 7000, 40
+// heads, took 41 us with them and take 242).
 //   S^T = K Q^T   A = K rows (16-byte LDS reads), B = q * scale * log2(e) as bf16 hi + lo (registers)
-//   softmax in base 2 (exp2), per query column (lane exchanges for the tile's max; the sums stay per lane
-//                 until the end, and the outputs are rescaled only where a max grew)
+//   softmax in base 2 (exp2), per query column (lane exchanges for the tile's max and sum; the outputs are
+//                 rescaled only where a max grew)
 //   O^T += V^T P^T  B = P^T from the S^T accumulators (hi + lo bf16: hardware conversions);
 //                 A = V^T read with the LDS transpose read: lane j of a 16-lane group reads key
 //                 base + (j >> 2), dims 4 (j & 3) .. + 3, and lane i receives dim i of the four
@@ -35,8 +35,8 @@ typedef float ff32x4_t __attribute__((ext_vector_type(4)));
 // 1.7. The page number and the position go through readfirstlane, or each copy becomes a loop over lanes whose
 // buffer descriptors might differ (2048 tokens after 28000: 2990 us so, 2310 now), and whole tiles have a loop
 // of their own, without masks and without a branch around each V fragment (130 -> 126 us at 2048 after 0).
-// 1000 tokens after 7001, 40 / 8 heads: 500 us with eight items of two query blocks per workgroup in one
-// range (one workgroup per CU), 412 in this cut, 317 in four ranges.
+// 1000 tokens after 7001, 40 / 8 heads: 475 us with eight items of two query blocks per workgroup (one
+// workgroup per CU), 379 in this cut.
 typedef short fp_v4s __attribute__((ext_vector_type(4)));
 typedef __bf16 fp_bf2 __attribute__((ext_vector_type(2)));
 typedef __attribute__((address_space(3))) void* fp_lptr;
@@ -54,8 +54,7 @@ __device__ __forceinline__ void split2(float x0, float x1, uint32_t& hi, uint32_
 
 struct FlashDev {
     FlashArgs a;
-    int nb, nwg, nsplit, first;   // query blocks, workgroups per KV head and key range, key ranges, ranks dealt heaviest first
-    float* po; float* pml;        // nsplit > 1: partial outputs [split][T][nH][128], (max, sum) [split][T][nH][2]
+    int nb, nwg, first;   // query blocks, workgroups per KV head, ranks dealt heaviest first
 };
 
 __global__ __launch_bounds__(256, 2) void flash_kernel(FlashDev f) {
@@ -64,9 +63,9 @@ __global__ __launch_bounds__(256, 2) void flash_kernel(FlashDev f) {
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int G = a.nH / a.nKV;
-    // KV heads fastest (with eight of them an XCD keeps to one), then key ranges, then item ranks: heaviest
-    // first, the ones past `first` lightest first (they share a CU with the heaviest)
-    const int per = a.nKV * f.nsplit, g = (int)blockIdx.x, rank = g / per, kvh = g % per % a.nKV, z = g % per / a.nKV;
+    // KV heads fastest (with eight of them an XCD keeps to one), then item ranks: heaviest first, the ones
+    // past `first` lightest first (they share a CU with the heaviest)
+    const int g = (int)blockIdx.x, rank = g / a.nKV, kvh = g % a.nKV;
     const int w = rank < f.first ? f.nwg - 1 - rank : rank - f.first;
     const int items = G * f.nb, item = 4 * w + wave, last = min(4 * w + 3, items - 1);
     const bool active = item < items;
@@ -74,9 +73,8 @@ __global__ __launch_bounds__(256, 2) void flash_kernel(FlashDev f) {
     const int pos0 = __builtin_amdgcn_readfirstlane(*a.dpos);
     const int q0 = blk * 32, nq = min(32, a.T - q0);
     const int kend = pos0 + q0 + nq;                                      // this wave's keys [0, kend)
-    const int all = (pos0 + min(last / G * 32 + 32, a.T) + 63) / 64;      // the last item's tiles, of which this range's:
-    const int tile0 = all * z / f.nsplit, tile1 = all * (z + 1) / f.nsplit;
-    const int ntiles = active ? min((kend + 63) / 64, tile1) : 0;
+    const int all = (pos0 + min(last / G * 32 + 32, a.T) + 63) / 64;      // the last item's tiles
+    const int ntiles = active ? (kend + 63) / 64 : 0;
     const int r16 = lane & 15, kq = lane >> 4;
     const float qscale = a.scale * 1.4426950408889634f;   // scores in base-2 units
 
@@ -176,22 +174,24 @@ __global__ __launch_bounds__(256, 2) void flash_kernel(FlashDev f) {
                 }
             mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
             mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+            float alpha = 1.0f;
             if (__any(mx > m[qb])) {
-                const float mn = fmaxf(m[qb], mx), alpha = mn == -INFINITY ? 1.0f : __builtin_amdgcn_exp2f(m[qb] - mn);
-                l[qb] *= alpha;
+                const float mn = fmaxf(m[qb], mx);
+                alpha = mn == -INFINITY ? 1.0f : __builtin_amdgcn_exp2f(m[qb] - mn);
                 m[qb] = mn;
 #pragma unroll
                 for (int n = 0; n < 8; n++) o[n][qb] *= alpha;
             }
             const float ms = m[qb] == -INFINITY ? 0.0f : m[qb];   // no key yet: every p is 2^-inf
-            float p[4][4];
+            float p[4][4], sum = 0.0f;
 #pragma unroll
             for (int kb = 0; kb < 4; kb++)
 #pragma unroll
                 for (int i = 0; i < 4; i++) {
                     p[kb][i] = __builtin_amdgcn_exp2f(s[kb][qb][i] - ms);
-                    l[qb] += p[kb][i];
+                    sum += p[kb][i];
                 }
+            l[qb] = l[qb] * alpha + xor32_sum(xor16_sum(sum));
             // k-slots of PV step st: 0..3 = keys 16 (2 st) + 4 kq + i, 4..7 = keys 16 (2 st + 1) + 4 kq + i
 #pragma unroll
             for (int st = 0; st < 2; st++) {
@@ -242,62 +242,31 @@ __global__ __launch_bounds__(256, 2) void flash_kernel(FlashDev f) {
         __builtin_amdgcn_sched_barrier(0);
     };
 
-    if (tile0 < tile1) issue(tile0);
+    issue(0);
     auto next = [&](int t) {
         __builtin_amdgcn_s_waitcnt(0);       // this wave's copies of tile t landed ...
         __builtin_amdgcn_s_barrier();        // ... and every wave's; tile t - 1's stage is free
-        if (t + 1 < tile1) issue(t + 1);
+        if (t + 1 < all) issue(t + 1);
     };
     // whole tiles: every key of theirs is at or before the block's first query
-    const int whole = max(tile0, min(ntiles, (pos0 + q0 + 1) / 64));
-    int t = tile0;
+    const int whole = min(ntiles, (pos0 + q0 + 1) / 64);
+    int t = 0;
     for (; t < whole; t++) { next(t); tile(std::false_type{}, t); }
     for (; t < ntiles; t++) { next(t); tile(std::true_type{}, t); }
-    for (; t < tile1; t++) next(t);
+    for (; t < all; t++) next(t);
     if (!active) return;
 #pragma unroll
     for (int qb = 0; qb < 2; qb++) {
-        float sum = l[qb];
-        sum += __shfl_xor(sum, 16, 64);
-        sum += __shfl_xor(sum, 32, 64);
         const int t = q0 + 16 * qb + r16;
         if (t >= a.T) continue;
-        const bool parts = f.nsplit > 1;
-        const size_t row = ((size_t)z * a.T + t) * a.nH + h;
-        const float inv = parts ? 1.0f : 1.0f / sum;
-        float* op = (parts ? f.po + row * 128 : a.out + (size_t)t * a.out_stride + (size_t)h * 128) + 4 * kq;
-        if (parts && kq == 0) *reinterpret_cast<float2*>(f.pml + 2 * row) = float2{m[qb], sum};
+        const float inv = 1.0f / l[qb];
+        float* op = a.out + (size_t)t * a.out_stride + (size_t)h * 128 + 4 * kq;
 #pragma unroll
         for (int n = 0; n < 8; n++)
             *reinterpret_cast<float4*>(op + 16 * n) = float4{o[n][qb][0] * inv, o[n][qb][1] * inv, o[n][qb][2] * inv, o[n][qb][3] * inv};
     }
 }
 
-// One wave per (token, head): the key ranges' partial outputs, weighted by 2^(max - largest max), in order.
-__global__ __launch_bounds__(256) void flash_merge_kernel(FlashDev f) {
-    const FlashArgs& a = f.a;
-    const int lane = threadIdx.x & 63, i = (int)blockIdx.x * 4 + (threadIdx.x >> 6), n = a.T * a.nH;
-    if (i >= n) return;
-    const float2 ml = lane < f.nsplit ? *reinterpret_cast<const float2*>(f.pml + 2 * ((size_t)lane * n + i)) : float2{-INFINITY, 0.0f};
-    const float M = wave_max(ml.x), wt = ml.x == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(ml.x - M);
-    const float inv = 1.0f / wave_sum(wt * ml.y);
-    float2 o = {0.0f, 0.0f};
-    for (int z = 0; z < f.nsplit; z += 8) {
-        float2 v[8];
-#pragma unroll
-        for (int j = 0; j < 8; j++) v[j] = *reinterpret_cast<const float2*>(f.po + ((size_t)min(z + j, f.nsplit - 1) * n + i) * 128 + 2 * lane);
-#pragma unroll
-        for (int j = 0; j < 8; j++)
-            if (z + j < f.nsplit) {
-                const float wz = __shfl(wt, z + j, 64);
-                o.x += v[j].x * wz; o.y += v[j].y * wz;
-            }
-    }
-    float* op = a.out + (size_t)(i / a.nH) * a.out_stride + (size_t)(i % a.nH) * 128 + 2 * lane;
-    op[0] = o.x * inv; op[1] = o.y * inv;
-}
-
-static int flash_workgroups(const FlashArgs& a) { return (a.nH / a.nKV * ((a.T + 31) / 32) + 3) / 4 * a.nKV; }
 static int flash_cus() {
     static std::atomic<int> cus{0};
     if (int c = cus.load(std::memory_order_relaxed)) return c;
@@ -305,51 +274,15 @@ static int flash_cus() {
     if (hipGetDevice(&dev) == hipSuccess && hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && n > 0) cus = n;
     return n > 0 ? n : 256;
 }
-// Key ranges by expected time. A workgroup alone on its CU takes 1.95 us a tile, two of them 3.45 us a tile
-// each (so pairs gain 1.13x, and a launch of fewer than a workgroup per CU gains the whole cut); the merge
-// reads and writes the partial outputs at ~3 TB/s behind a launch of ~5 us. The model is within 15% of the
-// times measured for 1 .. 32 ranges on 18 shapes (16 .. 2048 tokens after 0 .. 28000, 2 .. 40 heads), of
-// which it takes ranges for all but the first chunks with a workgroup per CU or more: 2048 tokens at 0, 32
-// heads, are 78 us in one range and 98 in two; 16 tokens after 7000, 40 heads, are 216 and 19 in sixteen.
-static int flash_splits(const FlashArgs& a, size_t part_floats) {
-    constexpr float ALONE = 1.95f, PAIR = 3.45f;
-    const int cus = flash_cus(), wgs = flash_workgroups(a);
-    const float tmax = float((a.pos + a.T + 63) / 64), tmin = float((a.pos + std::min(a.T, 32) + 63) / 64), avg = 0.5f * (tmin + tmax);
-    int best = 1;
-    float bestus = 0.0f;
-    for (int ns = 1; ns <= 32 && 2 * ns <= std::max(2.0f, tmax); ns++) {
-        if (ns > 1 && (size_t)ns * a.T * a.nH * 130 > part_floats) break;
-        const float n = (float)wgs * ns;
-        float us;
-        if (n <= cus) us = ceilf(tmax / ns) * ALONE;
-        else if (n <= 2 * cus) us = (tmin * PAIR + (tmax - tmin) * ALONE) / ns;   // heaviest beside lightest
-        else {
-            const float rounds = floorf(n / (2 * cus)), rest = n - rounds * 2 * cus;
-            us = (rounds * PAIR + (rest == 0 ? 0.0f : rest <= cus ? ALONE : PAIR)) * avg / ns;
-        }
-        if (ns > 1) us += 5.0f + (float)a.T * a.nH * ns * (2 * 520 / 3e6f);
-        if (ns == 1 || us < bestus) { best = ns; bestus = us; }
-    }
-    return best;
-}
-size_t flash_part_floats(const FlashArgs& a) {
-    const int ns = flash_splits(a, FLASH_PART_FLOATS);
-    return ns > 1 ? (size_t)ns * a.T * a.nH * 130 : 0;
-}
-
 hipError_t launch_flash_prefill(const FlashArgs& a, hipStream_t s) {
     if (a.D != 128 || a.nKV < 1 || a.nH % a.nKV || a.nH / a.nKV > 8 || a.T < 1) return hipErrorInvalidValue;
-    const int cus = flash_cus();
     FlashDev f{};
     f.a = a;
     f.nb = (a.T + 31) / 32;
-    f.nwg = flash_workgroups(a) / a.nKV;
-    f.nsplit = flash_splits(a, a.part ? a.part_floats : 0);
-    const int total = f.nwg * a.nKV * f.nsplit;
-    f.first = total > cus && total <= 2 * cus ? cus / (a.nKV * f.nsplit) : f.nwg;
-    if (f.nsplit > 1) { f.po = a.part; f.pml = a.part + (size_t)f.nsplit * a.T * a.nH * 128; }
+    f.nwg = (a.nH / a.nKV * f.nb + 3) / 4;
+    const int cus = flash_cus(), total = f.nwg * a.nKV;
+    f.first = total > cus && total <= 2 * cus ? cus / a.nKV : f.nwg;
     hipLaunchKernelGGL(flash_kernel, dim3(total), dim3(256), 4 * F2_TILE, s, f);
-    if (f.nsplit > 1) hipLaunchKernelGGL(flash_merge_kernel, dim3((a.T * a.nH + 3) / 4), dim3(256), 0, s, f);
     return hipGetLastError();
 }
 

@@ -140,11 +140,7 @@ struct FlashArgs {
     int D = 128, nH = 0, nKV = 0, T = 0;
     const int* dpos = nullptr;
     float scale = 1.0f;
-    int pos = 0;                        // *dpos as the host knows it: for the launch's cut only
-    float* part = nullptr; size_t part_floats = 0;   // optional scratch for key ranges (T nH 130 floats each)
 };
-constexpr size_t FLASH_PART_FLOATS = (size_t)1 << 24;    // most that a launch makes use of
-size_t flash_part_floats(const FlashArgs& a);            // what this one would (a.part not looked at)
 hipError_t launch_flash_prefill(const FlashArgs& a, hipStream_t s);
 
 hipError_t launch_silu_mul(const float* gu, float* out, int I, int T, hipStream_t s);

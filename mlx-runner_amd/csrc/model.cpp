@@ -603,7 +603,7 @@ int model_open(const char* dir_c, int context_len, const mlxr_sparse_cfg* sparse
         (rc = dalloc(m, &m->tmp, (size_t)2 * B * H)) || (rc = dalloc(m, &m->qkv, (size_t)2 * B * m->qkv_cols)) ||
         (rc = dalloc(m, &m->attn, (size_t)B * c.nH * c.D)) || (rc = dalloc(m, &m->gu, (size_t)B * 2 * I)) ||
         (rc = dalloc(m, &m->mlp, (size_t)B * I)) || (rc = dalloc(m, &m->logits, (size_t)8 * V)) || (rc = dalloc(m, &m->dmv_split, dpack_mv_split_floats(H))) ||
-        (rc = dalloc(m, &m->part, partFloats)) || (rc = dalloc(m, &m->qsplit, QGEMM_SPLIT_FLOATS)) || (rc = dalloc(m, &m->flash_part, FLASH_PART_FLOATS)) || (rc = dalloc(m, &m->bmax, (V + 255) / 256)) ||
+        (rc = dalloc(m, &m->part, partFloats)) || (rc = dalloc(m, &m->qsplit, QGEMM_SPLIT_FLOATS)) || (rc = dalloc(m, &m->bmax, (V + 255) / 256)) ||
         (rc = dalloc(m, &m->barg, (V + 255) / 256)) || (rc = dalloc(m, &m->xbf, (size_t)B * Kmax)) || (rc = dalloc(m, &m->xsc, (size_t)B)) || (rc = dalloc(m, &m->diag, 8)) ||
         (rc = dalloc(m, &m->xlo, (size_t)B * Kmax)) || (rc = dalloc(m, &m->xgs, qgemm_gsum_floats(B, Kmax, 32))) || (rc = dalloc(m, &m->xnz, (size_t)B)) || (rc = dalloc(m, &m->wsb, wsb_halves)))
         return fail(rc);
@@ -793,8 +793,7 @@ int attend(Model* m, int li, int T, Parts qkv_parts = Parts{}) {
     if (T > 8) {   // prefill chunk: flash attention on the matrix cores
         FlashArgs fa; fa.q = m->qkv; fa.q_stride = m->qkv_cols; fa.kc = ly.kc; fa.vc = ly.vc; fa.pt = m->page_table;
         fa.out = m->attn; fa.out_stride = c.nH * c.D; fa.D = c.D; fa.nH = c.nH; fa.nKV = c.nKV; fa.T = T;
-        fa.dpos = m->dpos; fa.scale = scale; fa.pos = std::max(0, m->dev_pos_known);
-        fa.part = m->flash_part; fa.part_floats = FLASH_PART_FLOATS;
+        fa.dpos = m->dpos; fa.scale = scale;
         HIPCHECK(launch_flash_prefill(fa, s));
     } else {       // verify batch: every query of a KV head in one pass over each key range
         AttnArgs aa; aa.q = m->qkv; aa.q_stride = m->qkv_cols; aa.kc = ly.kc; aa.vc = ly.vc; aa.pt = m->page_table;

@@ -65,7 +65,7 @@ struct Model {
     float* mm_split = nullptr;       // input-slice scratch of the verify batch's small-batch matvec (dpack_mm_split_floats)
     size_t mm_split_floats = 0;
     float* dmv_split = nullptr;      // [2][H] input-slice partials of the kernel-per-op down matvec (long inputs)
-    float* logits = nullptr; float* part = nullptr; float* flash_part = nullptr; float* bmax = nullptr; int* barg = nullptr;
+    float* logits = nullptr; float* part = nullptr; float* bmax = nullptr; int* barg = nullptr;
     float* qsplit = nullptr;            // the other widths' prefill GEMM split over K (QGEMM_SPLIT_FLOATS, counters at zero)
     uint16_t* xbf = nullptr; float* xsc = nullptr;
     uint16_t* xlo = nullptr; float* xgs = nullptr; int* xnz = nullptr;   // the MLX-layout GEMM's x lo part, group sums, lo flags

@@ -744,13 +744,11 @@ def test_flash_prefill(gpu, nH, nKV, offset, T):
 
 
 @pytest.mark.parametrize("nH,nKV,offset,T", [(2, 2, 3000, 33), (5, 1, 2040, 16), (16, 2, 4095, 9), (6, 2, 1999, 77), (40, 8, 900, 40)])
-def test_flash_key_ranges(gpu, nH, nKV, offset, T):
-    """Short chunks after a long context, whose keys the launch cuts into ranges merged afterwards: item
-    counts that are no multiple of four (3 heads x 3 blocks, 5 x 1, 1 x 2), ranges that end before a
-    block's last key or hold none of its keys, a last tile of one key and of 64, NaN past the last key.
-    A few tokens against the reference attention, 1e-4 relative (q and p as hi + lo bf16 pairs, ~2^-16,
-    fp32 sums; the merge adds at most 32 fp32 terms). One token's query is a multiple of one key, whose
-    range then outweighs the others."""
+def test_flash_after_context(gpu, nH, nKV, offset, T):
+    """Short chunks after a long context: item counts that are no multiple of four (3 heads x 3 blocks, 5 x 1,
+    1 x 2), a last tile of one key and of 64, NaN past the last key. A few tokens against the reference
+    attention, 1e-4 relative (q and p as hi + lo bf16 pairs, ~2^-16, fp32 sums). One token's query is a
+    multiple of one key, which then outweighs the others."""
     D, S = 128, (offset + T + 127) // 64 * 64
     rng = np.random.default_rng(nH + T)
     kc = bf16_to_f32(bf16_round(rng.uniform(-1, 1, (nKV, S, D)).astype(np.float32)))
@@ -766,6 +764,23 @@ def test_flash_key_ranges(gpu, nH, nKV, offset, T):
     for t in sorted({0, 1, T // 2, T - 2, T - 1}):
         ref = oracle.attention(q[t], kref, vref, nH, nKV, offset + t, scale)
         assert max_rel_err(got[t], ref) < 1e-4, (t, max_rel_err(got[t], ref))
+
+
+@pytest.mark.parametrize("nH,nKV,offset", [(16, 2, 1990), (40, 8, 64), (5, 1, 3001), (4, 4, 0)])
+def test_flash_is_chunk_invariant(gpu, nH, nKV, offset):
+    """A query's output has the same bits whatever chunk it arrives in: one call over 300 tokens against calls
+    over its pieces (of one token, less than a block of 32, across blocks), every row."""
+    D, T = 128, 300
+    S = (offset + T + 63) // 64 * 64
+    rng = np.random.default_rng(nH + offset)
+    kc = bf16_to_f32(bf16_round(rng.uniform(-1, 1, (nKV, S, D)).astype(np.float32)))
+    vc = bf16_to_f32(bf16_round(rng.uniform(-1, 1, (nKV, S, D)).astype(np.float32)))
+    q = rng.uniform(-1, 1, (T, nH, D)).astype(np.float32)
+    scale = 3 / np.sqrt(D)
+    whole = run_flash(gpu, q, kc, vc, nH, nKV, offset, T, scale).view(np.uint32)
+    for a, b in ((0, 9), (9, 40), (40, 41), (41, 170), (170, 300)):
+        got = run_flash(gpu, q[a:b], kc, vc, nH, nKV, offset + a, b - a, scale)
+        assert np.array_equal(got.view(np.uint32), whole[a:b]), (a, b)
 
 
 @pytest.mark.parametrize("nH,nKV", [(4, 2), (8, 2), (10, 2)])
