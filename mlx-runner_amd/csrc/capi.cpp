@@ -314,7 +314,7 @@ int mlxr_k_qgemm_tiles(const mlxr_qmat* parts, int nparts, int K, int gs, int ga
     if (int rc = ensure_buf(g_xbf, g_xbf_elems, (size_t)T * K)) { hipFree(code); return rc; }
     if (int rc = ensure_buf(g_xsc, g_xsc_elems, (size_t)T)) { hipFree(code); return rc; }
     hipError_t e = launch_x_to_f16(x, x_stride, K, T, g_xbf, g_xsc, g_stream);
-    if (e == hipSuccess) e = launch_tile_gemm(d, g_xbf, g_xsc, T, y, y_stride, tile_gemm_plan(d, T, 1), g_stream);
+    if (e == hipSuccess) e = launch_tile_gemm(d, g_xbf, g_xsc, T, y, y_stride, tile_gemm_plan(d, T), g_stream);
     const hipError_t e2 = hipStreamSynchronize(g_stream);
     hipFree(code);
     if (e == hipSuccess) e = e2;

@@ -26,11 +26,9 @@ hipError_t launch_dpack(const DPackSrc& s, uint8_t* out, hipStream_t st);
 // Prefill GEMM over a repacked matrix (ptile.hip): y[T][rows] (gated: y[T][o1] = SiLU(gate) * up)
 // from x already converted by the 4-bit GEMM pre-pass (xh: f16 rows scaled by 1 / inv[t]).
 bool tile_gemm_supported(const MvPhaseDesc& p);
-// How a tile GEMM is cut: 16 mi tokens x 8 rt row tiles per workgroup, K in S slices.
-struct TilePlan { int mi, rt, S; };
-TilePlan tile_gemm_plan(const MvPhaseDesc& p, int T, int max_slices);
-// S > 1: slice z's partial output at y + z * T * ys, to be added by the reader (a gated phase's slices
-// are the raw gate | up columns, ys >= 2 o1; with S == 1 its output is SiLU(gate) * up).
+// How a tile GEMM is cut: 16 mi tokens x 8 rt row tiles per workgroup. The output's bits don't depend on it.
+struct TilePlan { int mi, rt; };
+TilePlan tile_gemm_plan(const MvPhaseDesc& p, int T);
 hipError_t launch_tile_gemm(const MvPhaseDesc& p, const uint16_t* xh, const float* inv, int T, float* y, int ys, const TilePlan& plan,
                             hipStream_t s);
 

@@ -75,9 +75,6 @@ size_t qgemm_scale_halves(int O, int K, int gs);
 bool launch_row_f16(const float* x, int xs, int K, int T, uint16_t* out, float* inv, hipStream_t s);
 hipError_t launch_x_to_f16(const float* x, int xs, int K, int T, uint16_t* out, float* inv, hipStream_t s);
 
-// An input that is a sum of n partial outputs, stride floats apart (a GEMM's K slices), added in order.
-struct Parts { int n = 1; int64_t stride = 0; };
-
 // Embedding: out[t][k] = dequant(row ids[t]) (ids read from hist + *dpos + t0).
 hipError_t launch_qembed(const QMat& m, int K, int bits, int gs, int st, const int* hist, const int* dpos, int T,
                          float* out, hipStream_t s);
@@ -86,15 +83,12 @@ hipError_t launch_qembed(const QMat& m, int K, int bits, int gs, int st, const i
 hipError_t launch_rms_norm(const float* x, float* y, const float* w, int dim, int rows, int row_stride, float eps,
                            hipStream_t s);
 hipError_t launch_add_rms_norm(float* h, const float* r, float* y, const float* w, int dim, int rows, float eps,
-                               hipStream_t s, Parts rp = Parts{});
+                               hipStream_t s);
 // The same with the output in the 4-bit GEMM's f16 operand format (launch_x_to_f16's xh / inv).
 hipError_t launch_rms_norm_f16(const float* x, const float* w, int dim, int rows, int row_stride, float eps, uint16_t* xh,
                                float* inv, hipStream_t s);
 hipError_t launch_add_rms_norm_f16(float* h, const float* r, const float* w, int dim, int rows, float eps, uint16_t* xh,
-                                   float* inv, hipStream_t s, Parts rp = Parts{});   // rp.n > 1: dim <= ROW_F16_MAX
-// The down projection's operand from gate | up rows [T][2 I]: SiLU(gate) * up in the same format (I <= ROW_F16_MAX).
-hipError_t launch_silu_f16(const float* gu, int I, int T, uint16_t* out, float* inv, hipStream_t s, Parts rp);
-constexpr int ROW_F16_MAX = 32768;   // longest row of the single-pass operand kernels
+                                   float* inv, hipStream_t s);
 
 // Fused post-projection: per-head q/k RMSNorm, RoPE, q in place, K/V appended to the bf16 paged cache.
 struct QkvPostArgs {
@@ -107,9 +101,7 @@ struct QkvPostArgs {
     const int* dpos = nullptr; int pos_add = 0;
     float eps = 1e-6f;
     uint16_t* idx = nullptr;            // sparse block index: written for a block the step completes (T == 1)
-    Parts parts;                        // qkv as partial outputs (n > 1: where qkv_post_takes_parts)
 };
-bool qkv_post_takes_parts(int D, int rot_dim);
 hipError_t launch_qkv_post(const QkvPostArgs& a, hipStream_t s);
 
 // Decode attention (one query token per step, positions from *dpos + t): split over the keys,

@@ -45,26 +45,8 @@ __device__ __forceinline__ float block_sum_256(float v, float* red) {
     return t;
 }
 
-// Four consecutive values of a sum of partial outputs (rp.n of them, rp.stride floats apart, added in
-// order), NB loads in flight at a time, clamped ones past the last. Residual adds take 8 (up to 32
-// slices over 4096 values: 11.5 us one at a time, 8.0 by eight); gate | up rows, long and of few slices,
-// one (23 tokens, two slices: 12.9 us, 20.5 by eight).
-template <int NB>
-__device__ __forceinline__ float4 load_parts(const float* p, const Parts& rp) {
-    float4 v = *reinterpret_cast<const float4*>(p);
-    for (int z = 1; z < rp.n; z += NB) {
-        float4 u[NB];
-#pragma unroll
-        for (int j = 0; j < NB; j++) u[j] = *reinterpret_cast<const float4*>(p + min(z + j, rp.n - 1) * rp.stride);
-#pragma unroll
-        for (int j = 0; j < NB; j++)
-            if (z + j < rp.n) { v.x += u[j].x; v.y += u[j].y; v.z += u[j].z; v.w += u[j].w; }
-    }
-    return v;
-}
-
 __global__ __launch_bounds__(256) void rms_norm_kernel(const float* x, float* y, const float* w, int dim, int row_stride,
-                                                       float eps, int add, float* h, const float* r, Parts rp) {
+                                                       float eps, int add, float* h, const float* r) {
     __shared__ float red[4];
     const int row = blockIdx.x;
     float ss = 0.0f;
@@ -73,7 +55,7 @@ __global__ __launch_bounds__(256) void rms_norm_kernel(const float* x, float* y,
         const float* rr = r + (int64_t)row * row_stride;
         for (int i = threadIdx.x * 4; i < dim; i += 1024) {
             float4 v = *reinterpret_cast<float4*>(hr + i);
-            const float4 u = load_parts<8>(rr + i, rp);
+            const float4 u = *reinterpret_cast<const float4*>(rr + i);
             v.x += u.x; v.y += u.y; v.z += u.z; v.w += u.w;
             *reinterpret_cast<float4*>(hr + i) = v;
             ss += v.x * v.x + v.y * v.y + v.z * v.z + v.w * v.w;
@@ -161,35 +143,25 @@ __global__ __launch_bounds__(256) void rms_norm_f16_kernel(const float* x, const
 // rms_norm_f16_kernel with or without the residual add) for rows of up to 2048 NG values: each
 // thread loads its 8-groups g = tid + 256 i (i < NG) once, all loads in flight together, and keeps
 // them in registers through the reductions; the arithmetic per value is the same as those kernels'.
-// MODE 0: y = x; 1: y = RMSNorm(x) * w; 2: h += r (a sum of partial outputs), then y = RMSNorm(h) * w;
-// 3: y = SiLU(x[0 .. dim)) * x[dim .. 2 dim), both sums of partial outputs.
+// MODE 0: y = x; 1: y = RMSNorm(x) * w; 2: h += r, then y = RMSNorm(h) * w.
 template <int NG, int MODE>
 __global__ __launch_bounds__(256) void row_f16_kernel(const float* x, int row_stride, const float* w, int dim, float eps,
-                                                      float* h, const float* r, uint16_t* xh, float* invs, Parts rp) {
+                                                      float* h, const float* r, uint16_t* xh, float* invs) {
     __shared__ float red[4];
     const int row = blockIdx.x, ng = dim >> 3, tid = threadIdx.x;
     const float* xr = (MODE == 2 ? h : x) + (int64_t)row * row_stride;
-    auto silu = [](float g, float u) { return (g / (1.0f + expf(-g))) * u; };
     float4 v[NG][2], u[MODE == 2 ? NG : 1][2];
 #pragma unroll
     for (int i = 0; i < NG; i++) {
         const int g = tid + 256 * i;
         v[i][0] = v[i][1] = float4{0.0f, 0.0f, 0.0f, 0.0f};
         if (g < ng) {
-            if constexpr (MODE == 3) {
-#pragma unroll
-                for (int c = 0; c < 2; c++) {
-                    const float4 gt = load_parts<1>(xr + 8 * g + 4 * c, rp), up = load_parts<1>(xr + dim + 8 * g + 4 * c, rp);
-                    v[i][c] = float4{silu(gt.x, up.x), silu(gt.y, up.y), silu(gt.z, up.z), silu(gt.w, up.w)};
-                }
-            } else {
-                v[i][0] = *reinterpret_cast<const float4*>(xr + 8 * g);
-                v[i][1] = *reinterpret_cast<const float4*>(xr + 8 * g + 4);
-            }
+            v[i][0] = *reinterpret_cast<const float4*>(xr + 8 * g);
+            v[i][1] = *reinterpret_cast<const float4*>(xr + 8 * g + 4);
             if constexpr (MODE == 2) {
                 const float* rr = r + (int64_t)row * row_stride + 8 * g;
-                u[i][0] = load_parts<8>(rr, rp);
-                u[i][1] = load_parts<8>(rr + 4, rp);
+                u[i][0] = *reinterpret_cast<const float4*>(rr);
+                u[i][1] = *reinterpret_cast<const float4*>(rr + 4);
             }
         }
     }
@@ -207,7 +179,7 @@ __global__ __launch_bounds__(256) void row_f16_kernel(const float* x, int row_st
             *reinterpret_cast<float4*>(hr + 4) = v[i][1];
         }
     }
-    if constexpr (MODE == 1 || MODE == 2) {
+    if constexpr (MODE != 0) {
         float ss = 0.0f;
 #pragma unroll
         for (int i = 0; i < NG; i++) {
@@ -261,10 +233,10 @@ __global__ __launch_bounds__(256) void row_f16_kernel(const float* x, int row_st
 
 template <int MODE>
 static bool row_f16_launch(const float* x, int row_stride, const float* w, int dim, int rows, float eps, float* h,
-                           const float* r, uint16_t* xh, float* inv, hipStream_t s, Parts rp = Parts{}) {
+                           const float* r, uint16_t* xh, float* inv, hipStream_t s) {
     const int per = (dim / 8 + 255) / 256;
 #define MLXR_ROW_F16(NG)                                                                                         \
-    hipLaunchKernelGGL((row_f16_kernel<NG, MODE>), dim3(rows), dim3(256), 0, s, x, row_stride, w, dim, eps, h, r, xh, inv, rp)
+    hipLaunchKernelGGL((row_f16_kernel<NG, MODE>), dim3(rows), dim3(256), 0, s, x, row_stride, w, dim, eps, h, r, xh, inv)
     if (per <= 2) MLXR_ROW_F16(2);
     else if (per <= 4) MLXR_ROW_F16(4);
     else if (per <= 8) MLXR_ROW_F16(8);
@@ -277,10 +249,6 @@ static bool row_f16_launch(const float* x, int row_stride, const float* w, int d
 bool launch_row_f16(const float* x, int xs, int K, int T, uint16_t* out, float* inv, hipStream_t s) {
     return row_f16_launch<0>(x, xs, nullptr, K, T, 0.0f, nullptr, nullptr, out, inv, s);
 }
-hipError_t launch_silu_f16(const float* gu, int I, int T, uint16_t* out, float* inv, hipStream_t s, Parts rp) {
-    if (I % 8 || !row_f16_launch<3>(gu, 2 * I, nullptr, I, T, 0.0f, nullptr, nullptr, out, inv, s, rp)) return hipErrorInvalidValue;
-    return hipGetLastError();
-}
 
 hipError_t launch_rms_norm_f16(const float* x, const float* w, int dim, int rows, int row_stride, float eps, uint16_t* xh,
                                float* inv, hipStream_t s) {
@@ -291,10 +259,9 @@ hipError_t launch_rms_norm_f16(const float* x, const float* w, int dim, int rows
     return hipGetLastError();
 }
 hipError_t launch_add_rms_norm_f16(float* h, const float* r, const float* w, int dim, int rows, float eps, uint16_t* xh,
-                                   float* inv, hipStream_t s, Parts rp) {
+                                   float* inv, hipStream_t s) {
     if (dim % 8) return hipErrorInvalidValue;
-    if (row_f16_launch<2>(h, dim, w, dim, rows, eps, h, r, xh, inv, s, rp)) return hipGetLastError();
-    if (rp.n > 1) return hipErrorInvalidValue;
+    if (row_f16_launch<2>(h, dim, w, dim, rows, eps, h, r, xh, inv, s)) return hipGetLastError();
     hipLaunchKernelGGL(rms_norm_f16_kernel, dim3(rows), dim3(256), 0, s, (const float*)h, w, dim, dim, eps, 1, h, r, xh, inv);
     return hipGetLastError();
 }
@@ -302,12 +269,12 @@ hipError_t launch_add_rms_norm_f16(float* h, const float* r, const float* w, int
 hipError_t launch_rms_norm(const float* x, float* y, const float* w, int dim, int rows, int row_stride, float eps,
                            hipStream_t s) {
     hipLaunchKernelGGL(rms_norm_kernel, dim3(rows), dim3(256), 0, s, x, y, w, dim, row_stride, eps, 0, (float*)nullptr,
-                       (const float*)nullptr, Parts{});
+                       (const float*)nullptr);
     return hipGetLastError();
 }
 hipError_t launch_add_rms_norm(float* h, const float* r, float* y, const float* w, int dim, int rows, float eps,
-                               hipStream_t s, Parts rp) {
-    hipLaunchKernelGGL(rms_norm_kernel, dim3(rows), dim3(256), 0, s, (const float*)h, y, w, dim, dim, eps, 1, h, r, rp);
+                               hipStream_t s) {
+    hipLaunchKernelGGL(rms_norm_kernel, dim3(rows), dim3(256), 0, s, (const float*)h, y, w, dim, dim, eps, 1, h, r);
     return hipGetLastError();
 }
 
@@ -372,17 +339,6 @@ __global__ __launch_bounds__(256) void qkv_post_wave_kernel(QkvPostArgs a) {
     float* base = a.qkv + (int64_t)t * a.row_stride + (int64_t)h * 128;
     const int pos = *a.dpos + a.pos_add + t;
     float v0 = base[d0], v1 = base[d1];
-    for (int z = 1; z < a.parts.n; z += 8) {   // as load_parts
-        float u0[8], u1[8];
-#pragma unroll
-        for (int j = 0; j < 8; j++) {
-            const float* p = base + min(z + j, a.parts.n - 1) * a.parts.stride;
-            u0[j] = p[d0]; u1[j] = p[d1];
-        }
-#pragma unroll
-        for (int j = 0; j < 8; j++)
-            if (z + j < a.parts.n) { v0 += u0[j]; v1 += u1[j]; }
-    }
     if (h >= a.nH + a.nKV) {   // value head: straight to the cache
         const int64_t row = kv_row(a.pt, a.nKV, h - a.nH - a.nKV, pos) * 128;
         a.vc[row + d0] = f32_to_bf16(v0);
@@ -422,9 +378,7 @@ __global__ __launch_bounds__(256) void qkv_post_wave_kernel(QkvPostArgs a) {
     }
 }
 
-bool qkv_post_takes_parts(int D, int rot_dim) { return D == 128 && rot_dim == 128; }
 hipError_t launch_qkv_post(const QkvPostArgs& a, hipStream_t s) {
-    if (a.parts.n > 1 && !qkv_post_takes_parts(a.D, a.rot_dim)) return hipErrorInvalidValue;
     if (a.D == 128 && a.rot_dim == 128) {
         const int items = (a.nH + 2 * a.nKV) * a.T;
         hipLaunchKernelGGL(qkv_post_wave_kernel, dim3((items + 3) / 4), dim3(256), 0, s, a);

@@ -600,7 +600,7 @@ int model_open(const char* dir_c, int context_len, const mlxr_sparse_cfg* sparse
     int rc;
     if ((rc = dalloc(m, &m->hist, seq + 1)) || (rc = dalloc(m, &m->status, seq + 1)) || (rc = dalloc(m, &m->rng, 2)) ||
         (rc = dalloc(m, &m->dpos, 64)) || (rc = dalloc(m, &m->h, (size_t)B * H)) || (rc = dalloc(m, &m->xn, (size_t)B * H)) ||
-        (rc = dalloc(m, &m->tmp, (size_t)2 * B * H)) || (rc = dalloc(m, &m->qkv, (size_t)2 * B * m->qkv_cols)) ||
+        (rc = dalloc(m, &m->tmp, (size_t)B * H)) || (rc = dalloc(m, &m->qkv, (size_t)B * m->qkv_cols)) ||
         (rc = dalloc(m, &m->attn, (size_t)B * c.nH * c.D)) || (rc = dalloc(m, &m->gu, (size_t)B * 2 * I)) ||
         (rc = dalloc(m, &m->mlp, (size_t)B * I)) || (rc = dalloc(m, &m->logits, (size_t)8 * V)) || (rc = dalloc(m, &m->dmv_split, dpack_mv_split_floats(H))) ||
         (rc = dalloc(m, &m->part, partFloats)) || (rc = dalloc(m, &m->qsplit, QGEMM_SPLIT_FLOATS)) || (rc = dalloc(m, &m->bmax, (V + 255) / 256)) ||
@@ -770,23 +770,22 @@ int encode_decode(Model* m, const mlxr_sample_params* sp, bool sparse, bool logi
 // all_logits: logits of every row ([T][V], T <= 8); else of the last row only.
 // Prefill GEMM over a repacked phase: the f16 pre-pass of x (x == nullptr: the fused norm already
 // wrote m->xbf / m->xsc), then the tile GEMM.
-int project_tiles(Model* m, const MvPhaseDesc& p, const float* x, int xs, float* y, int ys, int T, const TilePlan& plan) {
+int project_tiles(Model* m, const MvPhaseDesc& p, const float* x, int xs, float* y, int ys, int T) {
     if (x) HIPCHECK(launch_x_to_f16(x, xs, p.K, T, m->xbf, m->xsc, m->stream));
-    HIPCHECK(launch_tile_gemm(p, m->xbf, m->xsc, T, y, ys, plan, m->stream));
+    HIPCHECK(launch_tile_gemm(p, m->xbf, m->xsc, T, y, ys, tile_gemm_plan(p, T), m->stream));
     return MLXR_OK;
 }
 
 // Attention of a batch's T queries (positions *dpos .. *dpos + T - 1) after their q|k|v: QK norms,
 // RoPE and the cache write, then flash attention (prefill chunks) or the split attention (verify
 // batches, T <= 8).
-int attend(Model* m, int li, int T, Parts qkv_parts = Parts{}) {
+int attend(Model* m, int li, int T) {
     const Config& c = m->cfg;
     hipStream_t s = m->stream;
     Layer& ly = m->layers[li];
     QkvPostArgs pa; pa.qkv = m->qkv; pa.row_stride = m->qkv_cols; pa.inv_freq = m->inv_freq; pa.kc = ly.kc; pa.vc = ly.vc;
     pa.pt = m->page_table; pa.qn = ly.q_norm; pa.kn = ly.k_norm; pa.D = c.D; pa.nH = c.nH; pa.nKV = c.nKV;
     pa.rot_dim = c.rot_dim; pa.traditional = c.traditional; pa.T = T; pa.dpos = m->dpos; pa.eps = c.eps;
-    pa.parts = qkv_parts;
     HIPCHECK(launch_qkv_post(pa, s));
     if (m->sparse_alloc) HIPCHECK(launch_sparse_index(ly.kc, m->page_table, ly.idx, c.nKV, c.D, m->dpos, 0, T, s));
     const float scale = c.query_scale * c.rope_attention_factor * c.rope_attention_factor;
@@ -849,49 +848,30 @@ int encode_batch(Model* m, int T, bool want_logits, bool all_logits) {
     if (small_tiles) return encode_verify(m, T, want_logits, all_logits);
     if (tiles) HIPCHECK(launch_rms_norm_f16(m->h, m->layers[0].in_norm, H, T, H, c.eps, m->xbf, m->xsc, s));
     else HIPCHECK(launch_rms_norm(m->h, m->xn, m->layers[0].in_norm, H, T, H, c.eps, s));
-    // the tile GEMMs' K slices: partial outputs side by side in each projection's own buffer (2 max_batch
-    // rows of q|k|v and of o / down, max_batch of gate|up), added by the kernel that reads it
-    const int fit = m->max_batch / T, fit2 = 2 * m->max_batch / T;
-    TilePlan pq{}, po{}, pd{}, pg{};   // the same for every layer: the shapes are
-    if (tiles) {
-        const LayerDev& d = m->tile_layers[0];
-        pq = tile_gemm_plan(d.qkv, T, qkv_post_takes_parts(c.D, c.rot_dim) ? fit2 : 1);
-        po = tile_gemm_plan(d.o, T, H <= ROW_F16_MAX ? fit2 : 1);
-        pg = tile_gemm_plan(d.gu, T, I <= ROW_F16_MAX ? fit : 1);
-        pd = tile_gemm_plan(d.down, T, H <= ROW_F16_MAX ? fit2 : 1);
-    }
     for (int li = 0; li < c.L; li++) {
         Layer& ly = m->layers[li];
-        const bool last = li + 1 == c.L;
-        if (tiles) {
-            const LayerDev& d = m->tile_layers[li];
-            auto parts = [&](const TilePlan& p, int ys) { return Parts{p.S, (int64_t)T * ys}; };
-            if (int rc = project_tiles(m, d.qkv, nullptr, H, m->qkv, m->qkv_cols, T, pq)) return rc;
-            if (int rc = attend(m, li, T, parts(pq, m->qkv_cols))) return rc;
-            if (int rc = project_tiles(m, d.o, m->attn, c.nH * c.D, m->tmp, H, T, po)) return rc;
-            HIPCHECK(launch_add_rms_norm_f16(m->h, m->tmp, ly.post_norm, H, T, c.eps, m->xbf, m->xsc, s, parts(po, H)));
-            if (pg.S > 1) {
-                if (int rc = project_tiles(m, d.gu, nullptr, H, m->gu, 2 * I, T, pg)) return rc;
-                HIPCHECK(launch_silu_f16(m->gu, I, T, m->xbf, m->xsc, s, parts(pg, 2 * I)));
-                if (int rc = project_tiles(m, d.down, nullptr, I, m->tmp, H, T, pd)) return rc;
-            } else {
-                if (int rc = project_tiles(m, d.gu, nullptr, H, m->mlp, I, T, pg)) return rc;
-                if (int rc = project_tiles(m, d.down, m->mlp, I, m->tmp, H, T, pd)) return rc;
-            }
-            if (!last) HIPCHECK(launch_add_rms_norm_f16(m->h, m->tmp, m->layers[li + 1].in_norm, H, T, c.eps, m->xbf, m->xsc, s, parts(pd, H)));
-            else if (want_logits) HIPCHECK(launch_add_rms_norm(m->h, m->tmp, m->xn, m->final_norm, H, T, c.eps, s, parts(pd, H)));
-            continue;
-        }
-        const Lin qkvp[3] = {ly.q, ly.k, ly.v}, gup[2] = {ly.gate, ly.up};
-        if (int rc = project(m, qkvp, 3, m->xn, H, m->qkv, m->qkv_cols, T)) return rc;
+        const Lin qkvp[3] = {ly.q, ly.k, ly.v};
+        const LayerDev* tl = tiles ? &m->tile_layers[li] : nullptr;
+        if (int rc = tl ? project_tiles(m, tl->qkv, nullptr, H, m->qkv, m->qkv_cols, T)
+                        : project(m, qkvp, 3, m->xn, H, m->qkv, m->qkv_cols, T)) return rc;
         if (int rc = attend(m, li, T)) return rc;
-        if (int rc = project(m, &ly.o, 1, m->attn, c.nH * c.D, m->tmp, H, T)) return rc;
-        HIPCHECK(launch_add_rms_norm(m->h, m->tmp, m->xn, ly.post_norm, H, T, c.eps, s));
-        if (int rc = project(m, gup, 2, m->xn, H, m->gu, 2 * I, T)) return rc;
-        HIPCHECK(launch_silu_mul(m->gu, m->mlp, I, T, s));
-        if (int rc = project(m, &ly.down, 1, m->mlp, I, m->tmp, H, T)) return rc;
+        if (int rc = tl ? project_tiles(m, tl->o, m->attn, c.nH * c.D, m->tmp, H, T)
+                        : project(m, &ly.o, 1, m->attn, c.nH * c.D, m->tmp, H, T)) return rc;
+        if (tl) {
+            HIPCHECK(launch_add_rms_norm_f16(m->h, m->tmp, ly.post_norm, H, T, c.eps, m->xbf, m->xsc, s));
+            if (int rc = project_tiles(m, tl->gu, nullptr, H, m->mlp, I, T)) return rc;
+        } else {
+            HIPCHECK(launch_add_rms_norm(m->h, m->tmp, m->xn, ly.post_norm, H, T, c.eps, s));
+            const Lin gup[2] = {ly.gate, ly.up};
+            if (int rc = project(m, gup, 2, m->xn, H, m->gu, 2 * I, T)) return rc;
+            HIPCHECK(launch_silu_mul(m->gu, m->mlp, I, T, s));
+        }
+        if (int rc = tl ? project_tiles(m, tl->down, m->mlp, I, m->tmp, H, T)
+                        : project(m, &ly.down, 1, m->mlp, I, m->tmp, H, T)) return rc;
+        const bool last = li + 1 == c.L;
         if (last && !want_logits) continue;
-        HIPCHECK(launch_add_rms_norm(m->h, m->tmp, m->xn, last ? m->final_norm : m->layers[li + 1].in_norm, H, T, c.eps, s));
+        if (tl && !last) HIPCHECK(launch_add_rms_norm_f16(m->h, m->tmp, m->layers[li + 1].in_norm, H, T, c.eps, m->xbf, m->xsc, s));
+        else HIPCHECK(launch_add_rms_norm(m->h, m->tmp, m->xn, last ? m->final_norm : m->layers[li + 1].in_norm, H, T, c.eps, s));
     }
     if (!want_logits) return MLXR_OK;
     if (all_logits) {

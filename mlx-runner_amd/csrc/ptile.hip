@@ -12,9 +12,9 @@
 // copy therefore reads 1 KB of consecutive bytes; copying the MLX layout instead (16-byte pieces of
 // 32 rows, 4-byte scale words) costs about three times the L1 accesses, which bounded the GEMM.
 //
-// Tile: a 512-thread workgroup owns 16 MI tokens x 8 RT DPack tiles (128 tokens x 256 rows: MI 8, RT 2)
-// and a slice of K (tile_gemm_plan picks the cut; a sliced launch leaves partial outputs that the kernel
-// reading them adds, in slice order: no counters, no extra launch). With RT 2, wave (wq, kc) computes the
+// Tile: a 512-thread workgroup owns 16 MI tokens x 8 RT DPack tiles (128 tokens x 256 rows: MI 8, RT 2;
+// tile_gemm_plan picks the cut). An output is one chain of products over all of K, in the same order in
+// every cut, so a token's result has the same bits in any batch. With RT 2, wave (wq, kc) computes the
 // tiles 4 wq + 2 kc, + 1 against all the tokens (MI X fragments x RT W fragments: 16 MFMAs per
 // 32-k step); two waves share each SIMD, so one issues MFMAs while the other waits on memory or
 // dequantizes. The X block (128 tokens x 128 k, f16, 16-byte chunks XOR-swizzled by (row & 15),
@@ -22,10 +22,10 @@
 // into three stages, two blocks ahead of the one being computed (one block ahead left about a third
 // of the waves' time waiting for the copies; where two workgroups share a CU, or 24 tiles leave no room,
 // two stages). Gated phases (gate rows in tile rows 0-7, up rows in 8-15) finish with SiLU(gate) * up in
-// the epilogue, so the MLP activation is written directly, unless K is sliced.
+// the epilogue, so the MLP activation is written directly.
 //
-// What bounds it: the matrix cores' issue at 128 tokens (2048 tokens: 0.9 PF/s), the weights' stream and
-// the launch itself at few (16 tokens, gate|up of the 8B shape: 66 MB in 21 us).
+// What bounds it: the matrix cores' issue at 128 tokens (2048 tokens: 0.9 PF/s); at few, each workgroup's
+// chain of blocks over K (0.93 us a block of 128 k).
 #include "decode.h"
 
 namespace mlxr {
@@ -51,7 +51,6 @@ struct TileGemmArgs {
     MvPhaseDesc p;
     const uint16_t* xh; const float* inv; float* y;
     int ys, T, nT, ntiles;               // ntiles: (token tile, row tile) pairs
-    int S; int64_t pstride;              // K slices; slice z's partial output at y + z * pstride
 };
 
 __device__ __forceinline__ half2_t bf16_half2(uint32_t raw16) {
@@ -59,8 +58,6 @@ __device__ __forceinline__ half2_t bf16_half2(uint32_t raw16) {
     return half2_t{h, h};
 }
 
-// GATED: 1: SiLU(gate) * up in the epilogue; 2 (a slice of a gated phase): the partial gate rows at
-// columns [0, o1), the up rows at [o1, 2 o1).
 template <int GATED, int MI, int RT, int NST, int OCC>
 __global__ __launch_bounds__(512, 2 * OCC) void tile_gemm_kernel(TileGemmArgs a) {
     constexpr int PT_M = 16 * MI, PT_XB = PT_M * 256;   // tokens; X block bytes
@@ -76,9 +73,8 @@ __global__ __launch_bounds__(512, 2 * OCC) void tile_gemm_kernel(TileGemmArgs a)
     // tile order: XCD x runs workgroups x, x + 8, ...; give it a contiguous run of tiles, and
     // enumerate tiles in columns of 8 row-tiles so that the ~32 workgroups an XCD runs at once cover
     // 4 token tiles x 8 row tiles (X and W blocks each shared in its L2 by several workgroups)
-    // K slices are the slowest index.
-    const int total = a.ntiles * a.S, g = blockIdx.x, xcd = g & 7, per = total >> 3, rem = total & 7;
-    const int item = xcd * per + min(xcd, rem) + (g >> 3), z = item / a.ntiles, tile = item - z * a.ntiles;
+    const int g = blockIdx.x, xcd = g & 7, per = a.ntiles >> 3, rem = a.ntiles & 7;
+    const int tile = xcd * per + min(xcd, rem) + (g >> 3);
     const int nO = a.ntiles / a.nT, ob = tile / (8 * a.nT), ow = min(8, nO - 8 * ob), r8 = tile - ob * 8 * a.nT;
     const int tt = r8 / ow, ot = 8 * ob + (r8 - tt * ow);
     const int t0 = ot * PT_TILES, m0 = tt * PT_M;
@@ -190,21 +186,19 @@ __global__ __launch_bounds__(512, 2 * OCC) void tile_gemm_kernel(TileGemmArgs a)
         __builtin_amdgcn_sched_barrier(0);
     };
 
-    const int b0 = nb * z / a.S, b1 = nb * (z + 1) / a.S;
-    issue(b0);
-    if (NST == 3 && b0 + 1 < b1) issue(b0 + 1);
-    for (int blk = b0; blk < b1; blk++) {
+    issue(0);
+    if (NST == 3 && nb > 1) issue(1);
+    for (int blk = 0; blk < nb; blk++) {
         // this wave's copies of block blk have landed (with three stages block blk + 1's may still
         // be in flight) ...
-        if (NST == 3 && blk + 1 < b1) __builtin_amdgcn_s_waitcnt(pt_wait_vm(NCP));
+        if (NST == 3 && blk + 1 < nb) __builtin_amdgcn_s_waitcnt(pt_wait_vm(NCP));
         else __builtin_amdgcn_s_waitcnt(0);
         // ... and every wave's; block blk + 1 - NST's stage, which block blk + NST - 1 overwrites,
         // is no longer read. A bare s_barrier: __syncthreads' fence adds nothing here.
         __builtin_amdgcn_s_barrier();
-        compute(blk, blk + NST - 1 < b1 ? blk + NST - 1 : -1);
+        compute(blk, blk + NST - 1 < nb ? blk + NST - 1 : -1);
     }
     // lane holds, for token m0 + 16 i + r16, rows 4 kq .. 4 kq + 3 of tile t0 + wt0 + u
-    float* const yz = a.y + z * a.pstride;
 #pragma unroll
     for (int u = 0; u < RT; u++) {
         const int t = t0 + wt0 + u;
@@ -213,25 +207,14 @@ __global__ __launch_bounds__(512, 2 * OCC) void tile_gemm_kernel(TileGemmArgs a)
             const int m = m0 + 16 * i + r16;
             const float iv = m < a.T ? a.inv[m] : 0.0f;
             f32x4_t v = acc[i][u] * iv;
-            if constexpr (GATED == 2) {
-                const int n = 8 * t + 4 * (kq & 1), part = kq >> 1;
-                if (m >= a.T || n >= a.p.o1) continue;
-                float* yp = yz + (int64_t)m * a.ys + part * a.p.o1 + n;
-                const uint16_t* bp = z == 0 ? a.p.bias[part] : nullptr;
-#pragma unroll
-                for (int r = 0; r < 4; r++)
-                    if (bp && n + r < a.p.o1) v[r] += bf16_to_f32(bp[n + r]);
-                if (n + 4 <= a.p.o1 && (reinterpret_cast<uintptr_t>(yp) & 15) == 0) *reinterpret_cast<f32x4_t*>(yp) = v;
-                else
-                    for (int r = 0; r < 4 && n + r < a.p.o1; r++) yp[r] = v[r];
-            } else if constexpr (GATED) {
+            if constexpr (GATED) {
                 // lanes kq < 2: gate rows 8t + 4kq + r; lanes kq >= 2: the matching up rows
                 const int n = 8 * t + 4 * (kq & 1);
                 f32x4_t up;
 #pragma unroll
                 for (int r = 0; r < 4; r++) up[r] = __shfl_xor(v[r], 32);
                 if (kq >= 2 || m >= a.T || n >= a.p.o1) continue;
-                float* yp = yz + (int64_t)m * a.ys + n;
+                float* yp = a.y + (int64_t)m * a.ys + n;
 #pragma unroll
                 for (int r = 0; r < 4; r++) {
                     float gt = v[r], ut = up[r];
@@ -244,14 +227,14 @@ __global__ __launch_bounds__(512, 2 * OCC) void tile_gemm_kernel(TileGemmArgs a)
             } else {
                 const int n = 16 * t + 4 * kq;
                 if (m >= a.T || n >= a.p.rows) continue;
-                float* yp = yz + (int64_t)m * a.ys + n;
+                float* yp = a.y + (int64_t)m * a.ys + n;
 #pragma unroll
                 for (int r = 0; r < 4; r++) {
                     const int nr = n + r;
                     const int part = nr < a.p.o1 ? 0 : nr < a.p.o1 + a.p.o2 ? 1 : 2;
                     const int row = nr - (part > 0 ? a.p.o1 : 0) - (part > 1 ? a.p.o2 : 0);
                     const uint16_t* bp = a.p.bias[part];
-                    if (bp && z == 0) v[r] += bf16_to_f32(bp[row]);
+                    if (bp) v[r] += bf16_to_f32(bp[row]);
                 }
                 if (n + 4 <= a.p.rows && (reinterpret_cast<uintptr_t>(yp) & 15) == 0) *reinterpret_cast<f32x4_t*>(yp) = v;
                 else
@@ -272,18 +255,15 @@ static hipError_t tile_gemm_launch(const TileGemmArgs& a0, hipStream_t s) {
     constexpr int lds = pt_lds_bytes<MI, RT, NST>();
     static bool attr = false;
     if (!attr) {
-        for (const void* f : {(const void*)tile_gemm_kernel<0, MI, RT, NST, OCC>, (const void*)tile_gemm_kernel<1, MI, RT, NST, OCC>,
-                              (const void*)tile_gemm_kernel<2, MI, RT, NST, OCC>})
+        for (const void* f : {(const void*)tile_gemm_kernel<0, MI, RT, NST, OCC>, (const void*)tile_gemm_kernel<1, MI, RT, NST, OCC>})
             if (hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, lds) != hipSuccess) return hipErrorInvalidValue;
         attr = true;
     }
     TileGemmArgs a = a0;
     a.nT = (a.T + 16 * MI - 1) / (16 * MI);
     a.ntiles = a.nT * ((a.p.tiles + 8 * RT - 1) / (8 * RT));
-    const dim3 grid(a.ntiles * a.S);
-    if (!a.p.gated) hipLaunchKernelGGL((tile_gemm_kernel<0, MI, RT, NST, OCC>), grid, dim3(512), lds, s, a);
-    else if (a.S == 1) hipLaunchKernelGGL((tile_gemm_kernel<1, MI, RT, NST, OCC>), grid, dim3(512), lds, s, a);
-    else hipLaunchKernelGGL((tile_gemm_kernel<2, MI, RT, NST, OCC>), grid, dim3(512), lds, s, a);
+    if (!a.p.gated) hipLaunchKernelGGL((tile_gemm_kernel<0, MI, RT, NST, OCC>), dim3(a.ntiles), dim3(512), lds, s, a);
+    else hipLaunchKernelGGL((tile_gemm_kernel<1, MI, RT, NST, OCC>), dim3(a.ntiles), dim3(512), lds, s, a);
     return hipGetLastError();
 }
 
@@ -299,35 +279,35 @@ static int device_cus() {
 // The cut with the least expected time. A workgroup of nb blocks takes a + nb * tb microseconds (fill
 // and epilogue, then one 128-k block after another); a CU that is given n of them takes n times that
 // where one fits (16 mi >= 128 tokens), and hides all but e of the next one's a where two do. Measured
-// over q|k|v, o, gate|up and down of the 8B shape, 16 .. 2048 tokens, 1 .. 16 slices: within ~10% of
-// these lines. Small launches take few tokens per workgroup and many slices (16 tokens, 4096 -> 6144
-// rows: 24 workgroups of 128 tokens 70 us, 192 of 16 tokens and an eighth of K 9.3 us; 14336 -> 4096
-// rows: 205 -> 13 us; 300 tokens, 4096 rows: 70 -> 25 us and 205 -> 54 us); long ones the largest tile
-// whose workgroups fill their rounds (2048 tokens, gate|up: 522 us with 16 row tiles, 493 with 24;
-// o: 79 and 103). A slice's partial output costs its reader one more pass over it.
-TilePlan tile_gemm_plan(const MvPhaseDesc& p, int T, int max_slices) {
+// over q|k|v, o, gate|up and down of the 8B shape, 16 .. 2048 tokens: within ~10% of these lines. Small
+// launches take few tokens per workgroup, long ones the largest tile whose workgroups fill their rounds
+// (2048 tokens, gate|up: 522 us with 16 row tiles, 493 with 24; o: 79 and 103). Whole prefills of four
+// layers of the 8B shape, 128 tokens per workgroup and by this choice: 16 tokens 1704 -> 1048 us, 65
+// 1820 -> 1116, 130 1930 -> 1233, 512 2345 -> 1788, 1000 3129 -> 2801, 2048 4807 -> 4685. K slices on
+// workgroups of their own, added by the kernel that reads the output, took 521 us at 16 tokens and 916 at
+// 130; but as many as fill the chip follow from T, and with them the order of a token's sums.
+TilePlan tile_gemm_plan(const MvPhaseDesc& p, int T) {
     struct Kind { int mi, rt, two; double a, tb, e; };
     static const Kind kinds[] = {{1, 2, 1, 5.5, 0.93, 2.0}, {2, 2, 1, 7.0, 1.0, 2.0}, {4, 2, 1, 9.0, 1.15, 3.0},
                                  {8, 2, 0, 10.0, 1.9, 0.0}, {8, 3, 0, 14.0, 2.5, 0.0}};
     const int cus = device_cus(), nb = p.K / PT_KB;
-    TilePlan best{8, 2, 1};
+    TilePlan best{8, 2};
     double bt = 1e30;
-    for (const Kind& k : kinds)
-        for (int S = 1; S <= 32 && S <= max_slices && (S == 1 || 2 * S <= nb); S++) {
-            const long wgs = (long)((T + 16 * k.mi - 1) / (16 * k.mi)) * ((p.tiles + 8 * k.rt - 1) / (8 * k.rt)) * S;
-            const double n = (double)((wgs + cus - 1) / cus), b = (double)((nb + S - 1) / S);
-            const double t = (k.two ? k.a + n * b * k.tb + (n - 1) * k.e : 3.0 + n * (k.a + b * k.tb)) + (S - 1) * (double)T * p.rows * 4 / 3e6;
-            if (t < bt) { bt = t; best = TilePlan{k.mi, k.rt, S}; }
-        }
+    for (const Kind& k : kinds) {
+        const long wgs = (long)((T + 16 * k.mi - 1) / (16 * k.mi)) * ((p.tiles + 8 * k.rt - 1) / (8 * k.rt));
+        const double n = (double)((wgs + cus - 1) / cus);
+        const double t = k.two ? k.a + n * nb * k.tb + (n - 1) * k.e : 3.0 + n * (k.a + nb * k.tb);
+        if (t < bt) { bt = t; best = TilePlan{k.mi, k.rt}; }
+    }
     return best;
 }
 
 hipError_t launch_tile_gemm(const MvPhaseDesc& p, const uint16_t* xh, const float* inv, int T, float* y, int ys, const TilePlan& plan,
                             hipStream_t s) {
-    if (!tile_gemm_supported(p) || T < 1 || plan.S < 1 || plan.S > p.K / PT_KB) return hipErrorInvalidValue;
+    if (!tile_gemm_supported(p) || T < 1 || plan.rt < 2 || plan.rt > 3 || (plan.rt == 3 && plan.mi != 8)) return hipErrorInvalidValue;
     TileGemmArgs a{};
-    a.p = p; a.xh = xh; a.inv = inv; a.y = y; a.ys = ys; a.T = T; a.S = plan.S; a.pstride = (int64_t)T * ys;
-    if (plan.mi == 8 && plan.rt == 3) return tile_gemm_launch<8, 3, 2, 1>(a, s);
+    a.p = p; a.xh = xh; a.inv = inv; a.y = y; a.ys = ys; a.T = T;
+    if (plan.rt == 3) return tile_gemm_launch<8, 3, 2, 1>(a, s);
     switch (plan.mi) {
         case 1: return tile_gemm_launch<1, 2, 3, 2>(a, s);
         case 2: return tile_gemm_launch<2, 2, 2, 2>(a, s);

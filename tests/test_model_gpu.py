@@ -203,11 +203,10 @@ def test_long_prefill_chunks(gpu, models):
 
 @pytest.mark.parametrize("name", ["qwen2", "qwen3_rope_half"])
 @pytest.mark.parametrize("n", [9, 16, 17, 33, 65, 129, 300])
-def test_prefill_tile_cuts_match_oracle(gpu, tmp_path, name, n):
-    """The prefill tile GEMM's cuts around their edges: 16 / 32 / 64 / 128 tokens per workgroup, K in
-    slices whose partial outputs the next kernel adds (qwen2: biases added once, gate | up slices; half
-    RoPE: a q|k|v reader that takes no slices). Every cut's logits at the gate against the oracle, or,
-    for the half RoPE that the oracle's model does not have, against the same tokens decoded one by one."""
+def test_short_prefills_match_oracle(gpu, tmp_path, name, n):
+    """Short and ragged prompts through the prefill tile GEMM (biases; half RoPE: the q|k|v reader of one
+    workgroup per head). Logits at the gate against the oracle, or, for the half RoPE that the oracle's
+    model does not have, against the same tokens decoded one by one."""
     cfg = configs.tiny("qwen2" if name == "qwen2" else "qwen3", tie=False, hidden=1024, inter=2048)
     if name != "qwen2":
         cfg = dict(cfg, partial_rotary_factor=0.5)
@@ -221,6 +220,27 @@ def test_prefill_tile_cuts_match_oracle(gpu, tmp_path, name, n):
                 exp = m.forward(toks[i:i + 1], i)
         got = m.forward(toks, 0)
         assert np.max(np.abs(got - exp)) < LOGIT_TOL
+
+
+@pytest.mark.parametrize("family,bits,gs", [("qwen2", 4, 64), ("qwen3", 4, 32), ("qwen3", 3, 32)])
+def test_prefill_is_chunk_invariant(gpu, tmp_path, family, bits, gs):
+    """A prompt leaves the same K/V bits and the same last logits whether it comes in one prefill or in
+    pieces of any length past 8 tokens (repacked tiles at 4 bits, MLX layout at 3): a second turn after a
+    reused prefix repeats the one-shot prompt."""
+    cfg = configs.tiny(family, bits=bits, gs=gs, tie=False, hidden=1024, inter=2048)
+    mlxr.synth_write(cfg, seed=bits, directory=str(tmp_path))
+    n, nkv, L = 700, cfg["num_key_value_heads"], cfg["num_hidden_layers"]
+    with mlxr.Transformer(str(tmp_path), context_length=1024) as m:
+        toks = prompt(n, m.vocab_size, seed=bits)
+        whole = m.forward(toks, 0).copy()
+        kv = [m.read_kv(i, n, nkv, 128) for i in range(L)]
+        for cuts in ((0, 9, 26, 59, 124, 253, 700), (0, 640, 700), (0, 300, 316, 700)):
+            for a, b in zip(cuts, cuts[1:]):
+                got = m.forward(toks[a:b], a)
+            for i in range(L):
+                for want, have in zip(kv[i], m.read_kv(i, n, nkv, 128)):
+                    assert np.array_equal(want.view(np.uint32), have.view(np.uint32)), (cuts, i)
+            assert np.array_equal(got.view(np.uint32), whole.view(np.uint32)), cuts
 
 
 def test_sparse_full_budget_is_bit_identical(gpu, models):
