@@ -41,7 +41,7 @@ struct QmmSmallArgs {
     float* split = nullptr; size_t split_floats = 0;   // optional scratch for K ranges, as QGemmArgs' (the same buffer serves both)
 };
 hipError_t launch_qmm_small(const QmmSmallArgs& a, hipStream_t s);
-bool qmb_supported(int gs);                             // group sizes of the matrix-core kernel; others run on the fp32 vector path
+bool qmb_supported(int K, int bits, int gs);            // shapes of the matrix-core kernel; others run on the fp32 vector path
 hipError_t launch_qmb(const QmmSmallArgs& a, hipStream_t s);
 
 // Prefill GEMM over the MLX layout, any code width: Y[T][O] = X[T][K] W[O][K]^T (+bias) with exact

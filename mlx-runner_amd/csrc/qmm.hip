@@ -99,10 +99,6 @@ __device__ __forceinline__ half8_t qb_codes(const uint32_t* d, int j) {
         v = gx_u4{qb_pair<3, 0>(e), qb_pair<3, 3>(e), qb_pair<3, 6>(e), qb_pair<3, 0>(e >> 9)};
     } else if constexpr (BITS == 4) {
         v = gx_u4{qb_pair<4, 0>(w0), qb_pair<4, 4>(w0), qb_pair<4, 0>(w0 >> 8), qb_pair<4, 4>(w0 >> 8)};
-    } else if constexpr (BITS == 5) {
-        const uint32_t t = __builtin_amdgcn_alignbit(w1, w0, 20);
-        const uint32_t e0 = __builtin_amdgcn_perm(t, w0, 0x05040100u), e1 = __builtin_amdgcn_perm(t, w0, 0x06050201u);
-        v = gx_u4{qb_pair<5, 0>(e0), qb_pair<5, 5>(e0), qb_pair<5, 2>(e1), qb_pair<5, 0>(e1 >> 7)};
     } else if constexpr (BITS == 6) {
         const uint32_t e0 = __builtin_amdgcn_perm(w1, w0, 0x04030100u), e1 = __builtin_amdgcn_perm(w1, w0, 0x05040201u);
         v = gx_u4{qb_pair<6, 0>(e0), qb_pair<6, 0>(e0 >> 6), qb_pair<6, 4>(e1), qb_pair<6, 0>(e1 >> 10)};
@@ -376,10 +372,18 @@ static int qb_cus() {
     return n > 0 ? n : 256;
 }
 
-bool qmb_supported(int gs) { return gs == 32 || gs == 64 || gs == 128; }
+// The shapes whose x goes to the matrix cores as f16 hi + lo: a value keeps 22 bits beside the largest of its
+// 1024 inputs, fewer the smaller it is beside that, and an infinity comes out as NaN. 5-bit codes, and 2, 3 and
+// 6 bits where K is no whole number of eight groups (four of 128 codes), hold x in fp32 and stay on the vector
+// path (4096 -> 14336 at 5 bits, T = 4: 43 us there, 23 here; 8320 -> 4096 at 3 bits: 31 and 17).
+bool qmb_supported(int K, int bits, int gs) {
+    if ((gs != 32 && gs != 64 && gs != 128) || K % gs) return false;
+    if (bits == 4 || bits == 8) return true;
+    return bits != 5 && K % ((gs == 128 ? 4 : 8) * gs) == 0 && K / gs <= 2048;
+}
 
 hipError_t launch_qmb(const QmmSmallArgs& a, hipStream_t s) {
-    if (!qmb_supported(a.gs) || a.T < 1 || a.T > 8) return hipErrorInvalidValue;
+    if (!qmb_supported(a.K, a.bits, a.gs) || a.T < 1 || a.T > 8) return hipErrorInvalidValue;
     QbDev d{};
     for (int i = 0; i < 3; i++) {
         const QMat& m = a.part[i < a.nparts ? i : a.nparts - 1];
@@ -391,7 +395,7 @@ hipError_t launch_qmb(const QmmSmallArgs& a, hipStream_t s) {
     // Tiles per wave and K ranges by expected time: a round of a workgroup per CU takes 2 us to start, 0.3 us a
     // chunk to convert x and 0.7 us a chunk and tile (a CU holds three or four workgroups, so later rounds
     // overlap a little); ranges add the hand-over, more with more partial sums. Over 120 shapes (512 .. 151936 rows,
-    // 1024 .. 28672 inputs, every width and group size, T = 2 .. 8) it takes 0.37 .. 1.0 of the former kernels'
+    // 1024 .. 28672 inputs, widths and group sizes, T = 2 .. 8) it takes 0.37 .. 1.0 of the former kernels'
     // time: 5120 -> 17000 with four tiles and seven ranges 22 us, with two tiles and one range 36.
     const bool split = a.split && a.split_floats >= QGEMM_SPLIT_FLOATS;
     int RT = 1, S = 1;
@@ -414,7 +418,7 @@ hipError_t launch_qmb(const QmmSmallArgs& a, hipStream_t s) {
         else hipLaunchKernelGGL((qmb_kernel<B, GS, 1>), grid, dim3(256), lds, s, d); \
         return hipGetLastError(); }
 #define QB_BITS(B) QB_GO(B, 32) QB_GO(B, 64) QB_GO(B, 128)
-    QB_BITS(2) QB_BITS(3) QB_BITS(4) QB_BITS(5) QB_BITS(6) QB_BITS(8)
+    QB_BITS(2) QB_BITS(3) QB_BITS(4) QB_BITS(6) QB_BITS(8)
 #undef QB_BITS
 #undef QB_GO
     return hipErrorInvalidValue;

@@ -171,7 +171,10 @@ def test_qmm_small_batch_cuts(gpu, bits, gs):
     sums of K / 32 products of 32 terms and of at most 16 ranges, x = hi + lo to 2^-21 of its slice's largest."""
     rng = np.random.default_rng(bits * 100 + gs)
     tail = 128 if gs == 128 else 64
-    for K, Os, T in ((8192 + 128, (33, 20, 17), 8), (8192 + 128, (8200,), 3), (256 + tail, (20000,), 5), (1024 + 128, (1,), 2), (tail, (65,), 7)):
+    shapes = [(8192 + 128, (33, 20, 17), 8), (8192 + 128, (8200,), 3), (256 + tail, (20000,), 5), (1024 + 128, (1,), 2), (tail, (65,), 7)]
+    if bits in (2, 3, 6):       # whole numbers of eight groups (four at gs 128): above, the fp32 vector path
+        shapes += [(8192 + 512, (33, 20, 17), 8), (8192 + 512, (8200,), 3), (512, (20000,), 5), (1536, (1,), 2), (512, (65,), 7)]
+    for K, Os, T in shapes:
         fxs = [QuantFixture(O, K, bits, gs, st="f16" if bits % 2 else "bf16", seed=O + K, with_bias=len(Os) > 1, fast=True) for O in Os]
         O, xs = sum(Os), K + 8
         qm = (gpu.QMat * len(fxs))(*[f.device(gpu) for f in fxs])
@@ -196,6 +199,43 @@ def test_qmm_small_batch_cuts(gpu, bits, gs):
                 tol = (K / 32 + 64) * 2.0**-24 * (top @ size) + 2.0**-21 * 2.0**-11 * (big @ size) + 1e-6
                 assert np.all(np.abs(got[:, col:col + f.O] - ref) <= tol), (K, Os, T)
                 col += f.O
+
+
+@pytest.mark.parametrize("bits,K,gs", [(5, 512, 64), (5, 8192, 128), (5, 1024, 32), (2, 576, 64), (3, 8320, 32), (6, 640, 128)])
+def test_qmm_small_batch_fp32_inputs(gpu, bits, K, gs):
+    """Shapes whose x stays in fp32 (5 bits; 2, 3 and 6 bits where K is no whole number of eight groups, four
+    at gs 128): values of 1e-3 beside one of 1e6 that meets zero weights, at a bound of fp32 sums alone; an
+    input of 3.2e38 (past the f16 scaling) and an infinity, each against codes of one."""
+    O, T, k0 = 21, 5, K // 2 + 3
+    fx = QuantFixture(O, K, bits, gs, seed=K, fast=True)
+    fx.s_raw[:, k0 // gs] = fx.b_raw[:, k0 // gs] = 0
+    fx.scales[:, k0 // gs] = fx.biases[:, k0 // gs] = 0
+    x = np.random.default_rng(K).normal(0, 1e-3, (T, K)).astype(np.float32)
+    x[1::2, k0] = 1e6
+
+    def run(x):
+        qm = (gpu.QMat * 1)(fx.device(gpu))
+        dx, dy = gpu.DeviceArray.from_numpy(x), gpu.DeviceArray.zeros((T, O), np.float32)
+        gpu.check(gpu.lib.mlxr_k_qmm(qm, 1, K, bits, gs, 0, T, dx.ptr, K, dy.ptr, O))
+        gpu.synchronize()
+        return dy.numpy()
+    g = np.repeat(np.arange(K // gs), gs)
+    w = fx.codes * fx.scales[:, g].astype(np.float64) + fx.biases[:, g]
+    size = np.abs(x).astype(np.float64) @ (fx.codes * np.abs(fx.scales[:, g]) + np.abs(fx.biases[:, g])).T
+    assert np.all(np.abs(run(x) - x.astype(np.float64) @ w.T) <= (K / 32 + 64) * 2.0**-24 * size)
+    fx.codes[:, g == k0 // gs] = 1
+    fx.packed = fx._pack_fast()
+    fx.scales[:, k0 // gs] = fx.biases[:, k0 // gs] = 2.0**-100
+    fx.s_raw[:, k0 // gs] = fx.b_raw[:, k0 // gs] = bf16_round(np.float32([2.0**-100]))[0]
+    x[:, g == k0 // gs] = 0
+    x[1, k0], x[3, k0] = 3.2e38, np.inf
+    got, small = run(x), x.copy()
+    small[:, k0] = 0
+    want = small.astype(np.float64) @ w.T
+    want[1] += 3.2e38 * 2.0**-99
+    ok = np.arange(T) != 3
+    assert np.all(np.abs(got[ok] - want[ok]) <= 1e-5 * (1 + np.abs(want[ok])))
+    assert np.all(got[3] == np.inf)
 
 
 def qgemm(mlxr, fx, x):
