@@ -6,6 +6,7 @@
 #include <string>
 #include <vector>
 #include "model.h"
+#include "scratch.h"
 
 namespace mlxr { int synth_write(const char* config_json, uint64_t seed, float std_, const char* dir); }
 
@@ -60,16 +61,12 @@ int ensure_pt(int max_seq) {
     return MLXR_OK;
 }
 template <typename T> int ensure_buf(T*& p, size_t& have, size_t need) {
-    if (need <= have) return MLXR_OK;
-    if (p) { hipStreamSynchronize(g_stream); hipFree(p); p = nullptr; have = 0; }
-    CK(hipMalloc(&p, need * sizeof(T)));
-    have = need;
+    CK(scratch_grow(p, have, need, g_stream));
     return MLXR_OK;
 }
-int ensure_qsplit() {
-    if (g_qsplit) return MLXR_OK;
-    if (int rc = ensure_buf(g_qsplit, g_qsplit_floats, QGEMM_SPLIT_FLOATS)) return rc;
-    CK(hipMemset(g_qsplit, 0, QGEMM_SPLIT_FLOATS * 4));
+hipError_t grow_qsplit() { return scratch_grow_zeroed(g_qsplit, g_qsplit_floats, QGEMM_SPLIT_FLOATS, QGEMM_SPLIT_TILES, g_stream); }
+int ensure_split(size_t need) {
+    CK(scratch_grow_zeroed(g_split, g_split_floats, need, DMV_SPLIT_CNT, g_stream));
     return MLXR_OK;
 }
 bool bits_ok(int b) { return b == 2 || b == 3 || b == 4 || b == 5 || b == 6 || b == 8; }
@@ -250,7 +247,7 @@ int mlxr_k_qmm(const mlxr_qmat* parts, int nparts, int K, int bits, int gs, int 
     QmmSmallArgs a; a.nparts = nparts;
     for (int i = 0; i < nparts; i++) a.part[i] = qmat(parts[i]);
     a.K = K; a.bits = bits; a.gs = gs; a.st = st; a.O = O; a.T = T; a.x = x; a.x_stride = x_stride; a.y = y; a.y_stride = y_stride;
-    if (ensure_qsplit() != MLXR_OK) (void)hipGetLastError();   // no room: no K ranges
+    if (qmb_supported(K, bits, gs) && grow_qsplit() != hipSuccess) (void)hipGetLastError();   // no room: no K ranges
     a.split = g_qsplit; a.split_floats = g_qsplit_floats;
     return done(launch_qmm_small(a, g_stream));
 }
@@ -267,7 +264,7 @@ int mlxr_k_qgemm(const mlxr_qmat* mat, int K, int bits, int gs, int st, int T, c
     if (int rc = ensure_buf(g_xgs, g_xgs_elems, qgemm_gsum_floats(T, K, gs))) return rc;
     if (int rc = ensure_buf(g_wsb, g_wsb_elems, qgemm_scale_halves(mat->O, K, gs))) return rc;
     if (int rc = ensure_buf(g_xnz, g_xnz_elems, (size_t)T)) return rc;
-    if (int rc = ensure_qsplit()) return rc;
+    CK(grow_qsplit());
     QGemmArgs a; a.m = qmat(*mat); a.K = K; a.bits = bits; a.gs = gs; a.st = st; a.O = mat->O; a.T = T;
     a.x = x; a.x_stride = x_stride; a.y = y; a.y_stride = y_stride; a.xbf = g_xbf; a.xsc = g_xsc;
     a.xlo = g_xlo; a.xgs = g_xgs; a.xnz = g_xnz; a.wsb = g_wsb;
@@ -330,11 +327,7 @@ int mlxr_k_qmv_tiles(const mlxr_qmat* parts, int nparts, int K, int gs, int mode
     if (int rc = tiles_pack(parts, nparts, K, gs, mode == 2, d, code)) return rc;
     if (!dpack_mv_supported(d)) { hipFree(code); return set_error(MLXR_E_UNSUPPORTED, "matvec over repacked tiles: K too large"); }
     // the scratch of the input-sliced matvec, as the model's kernel-per-op step passes it
-    const size_t sf = dpack_mv_split_floats(d.rows);
-    if (sf > g_split_floats) {
-        if (int rc = ensure_buf(g_split, g_split_floats, sf)) { hipFree(code); return rc; }
-        CK(hipMemset(g_split, 0, sf * 4));   // tile counters start at zero and return to it
-    }
+    if (int rc = ensure_split(dpack_mv_split_floats(d.rows))) { hipFree(code); return rc; }
     hipError_t e = hipSuccess;
     for (int r = 0; r < reps && e == hipSuccess; r++) e = launch_dpack_mv(d, x, norm_w, eps, y, mode, g_stream, g_split);
     const hipError_t e2 = hipStreamSynchronize(g_stream);
@@ -355,12 +348,8 @@ int mlxr_k_qmm_tiles(const mlxr_qmat* parts, int nparts, int K, int gs, int mode
     if (int rc = tiles_pack(parts, nparts, K, gs, mode == 2, d, code)) return rc;
     const int cols = mode == 2 ? d.o1 : d.rows;
     if (y_stride < cols) { hipFree(code); return set_error(MLXR_E_INVALID_ARG, "y_stride"); }
-    // the input-slice scratch, as the model passes it (tile counters start at zero and return to it)
-    const size_t sf = dpack_mm_split_floats(d);
-    if (sf > g_split_floats) {
-        if (int rc = ensure_buf(g_split, g_split_floats, sf)) { hipFree(code); return rc; }
-        CK(hipMemset(g_split, 0, sf * 4));
-    }
+    // the input-slice scratch, as the model passes it
+    if (int rc = ensure_split(dpack_mm_split_floats(d))) { hipFree(code); return rc; }
     hipError_t e = launch_dpack_mm(d, x, x_stride, norm_w, eps, y, y_stride, mode == 1, T, g_split, g_split_floats, g_stream);
     const hipError_t e2 = hipStreamSynchronize(g_stream);
     hipFree(code);

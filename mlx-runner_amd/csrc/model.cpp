@@ -641,6 +641,7 @@ int model_open(const char* dir_c, int context_len, const mlxr_sparse_cfg* sparse
     for (auto& s : m->slots) { HIPCHECK(hipEventCreate(&s.start)); HIPCHECK(hipEventCreate(&s.stop)); }
     if ((rc = model_seed(m, 0))) return fail(rc);
     if ((rc = tiles_setup(m)) || (rc = mega_setup(m))) return fail(rc);
+    HIPCHECK(hipDeviceSynchronize());   // the clears above ran on another stream than the model's
     *out = m;
     return MLXR_OK;
 }
