@@ -34,7 +34,7 @@ __device__ __forceinline__ void dmv_finish(const MvPhaseDesc& p, const MvLds& L,
         if (row >= p.rows) break;
         const float v = tile_row(L.part, i >> 4, i & 15, nfw, g.NF) * unscale + row_bias(p, row);
         if (MODE == OUT_ADD) y[row] += v;
-        else if (MODE == DMV_OUT_PARTIAL) __hip_atomic_store(y + row, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        else if (MODE == DMV_OUT_PARTIAL) part_store(y + row, v);
         else y[row] = v;
     }
 }
@@ -192,25 +192,22 @@ __global__ void __launch_bounds__(MK_THREADS) dpack_mv_split_kernel(MvPhaseDesc 
     q.tstride = NF;
     q.bias[0] = q.bias[1] = q.bias[2] = nullptr;
     dmv_body<FB, DMV_OUT_PARTIAL, true>(q, x + fa * FB * 128, nullptr, 0.0f, part + (size_t)sl * p.rows, tpw, w, nw);
-    // the partial rows are stored through to memory (agent scope) and waited for before the tiles' counters
-    // move, so the hand-over needs no write-back or invalidation of the caches (an acquire-release's)
-    __builtin_amdgcn_s_waitcnt(0);
-    __syncthreads();
+    parts_stored();
     __shared__ int last[MK_TPW];
     const MvGeom<FB> g = mv_geom<FB>(q, w, nw, 0);
     if ((int)threadIdx.x < g.nt)
-        last[threadIdx.x] = __hip_atomic_fetch_add(cnt + g.t0 + threadIdx.x, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == (unsigned)(S - 1);
+        last[threadIdx.x] = part_last(cnt + g.t0 + threadIdx.x, S);
     __syncthreads();
     for (int i = threadIdx.x; i < g.nt * 16; i += MK_THREADS) {
         if (!last[i >> 4]) continue;
         const int r = 16 * g.t0 + i;
         if (r < p.rows) {
             float v = 0.0f;
-            for (int k = 0; k < S; k++) v += __hip_atomic_load(part + (size_t)k * p.rows + r, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            for (int k = 0; k < S; k++) v += part_load(part + (size_t)k * p.rows + r);
             v += row_bias(p, r);
             y[r] = accumulate ? y[r] + v : v;
         }
-        if ((i & 15) == 0) __hip_atomic_store(cnt + g.t0 + (i >> 4), 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if ((i & 15) == 0) part_rearm(cnt + g.t0 + (i >> 4));
     }
 }
 
@@ -457,7 +454,7 @@ __global__ void __launch_bounds__(MK_THREADS) dpack_mm_kernel(MmArgs a) {
     // a finished row: to y (one slice) or to the slice's partials
     auto put = [&](int tl, int row, int tk, float v) {
         if (!direct) {
-            __hip_atomic_store(a.part + ((size_t)sl * nt + tk) * R + 16 * (T0 + tl) + row, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            part_store(a.part + ((size_t)sl * nt + tk) * R + 16 * (T0 + tl) + row, v);
             return;
         }
         const int r = 16 * (T0 + tl) + row;
@@ -512,19 +509,16 @@ __global__ void __launch_bounds__(MK_THREADS) dpack_mm_kernel(MmArgs a) {
         else put(tl, row, tk, v * unscale[tk]);
     }
     if (direct) return;
-    // the slices' partials are stored through to memory (agent scope) and waited for before the tiles' counters
-    // move (no write-back or invalidation of the caches, as an acquire-release would do);
-    // the tile's last workgroup sums them in slice order
-    __builtin_amdgcn_s_waitcnt(0);
-    __syncthreads();
+    // the tile's last workgroup sums the slices' partials in slice order
+    parts_stored();
     int* last = reinterpret_cast<int*>(slots);
     if ((int)threadIdx.x < g0.nt)
-        last[threadIdx.x] = __hip_atomic_fetch_add(a.cnt + T0 + threadIdx.x, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == (unsigned)(S - 1);
+        last[threadIdx.x] = part_last(a.cnt + T0 + threadIdx.x, S);
     __syncthreads();
     auto partial = [&](int tl, int row, int tk) {
         float v = 0.0f;
         for (int k = 0; k < S; k++)
-            v += __hip_atomic_load(a.part + ((size_t)k * nt + tk) * R + 16 * (T0 + tl) + row, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            v += part_load(a.part + ((size_t)k * nt + tk) * R + 16 * (T0 + tl) + row);
         return v;
     };
     for (int i = threadIdx.x; i < g0.nt * 16 * nt; i += MK_THREADS) {
@@ -550,7 +544,7 @@ __global__ void __launch_bounds__(MK_THREADS) dpack_mm_kernel(MmArgs a) {
         }
     }
     if ((int)threadIdx.x < g0.nt && last[threadIdx.x])
-        __hip_atomic_store(a.cnt + T0 + threadIdx.x, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        part_rearm(a.cnt + T0 + threadIdx.x);
 }
 
 template <int FB, int MODE>

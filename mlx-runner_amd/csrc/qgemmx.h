@@ -431,7 +431,7 @@ __device__ __forceinline__ void qgemmx_body(const QGemmXDev& a, uint8_t* lds, in
 #pragma unroll
                 for (int j = 0; j < J; j++)
 #pragma unroll
-                    for (int r = 0; r < 16; r++) __hip_atomic_store(a.part + pidx(sl, i, j, r), tot[i][j][r], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    for (int r = 0; r < 16; r++) part_store(a.part + pidx(sl, i, j, r), tot[i][j][r]);
         } else if (SF > 1) {
             // slices added in order, each from zero; their running sum waits in the thread's own outputs
             // (opaque indexes: addresses kept across the block loop would cost it its registers)
@@ -475,15 +475,12 @@ __device__ __forceinline__ void qgemmx_body(const QGemmXDev& a, uint8_t* lds, in
         }
     }
     if (a.S > 1) {
-        // the partial tile is stored through to memory (agent scope) and waited for before its counter moves: no
-        // write-back or invalidation of the caches (an acquire-release's)
-        __builtin_amdgcn_s_waitcnt(0);
-        __syncthreads();
+        parts_stored();
         __shared__ int last;
-        if (tid == 0) last = __hip_atomic_fetch_add(a.cnt + tile, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == (unsigned)(a.S - 1);
+        if (tid == 0) last = part_last(a.cnt + tile, a.S);
         __syncthreads();
         if (!last) return;
-        if (tid == 0) __hip_atomic_store(a.cnt + tile, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (tid == 0) part_rearm(a.cnt + tile);
         for (int sl = 0; sl < SF; sl++) {   // in order
 #pragma unroll
             for (int i = 0; i < I; i++)
@@ -491,7 +488,7 @@ __device__ __forceinline__ void qgemmx_body(const QGemmXDev& a, uint8_t* lds, in
                 for (int j = 0; j < J; j++) {
                     f32x16_t v;
 #pragma unroll
-                    for (int r = 0; r < 16; r++) v[r] = __hip_atomic_load(a.part + pidx(sl, i, j, r), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    for (int r = 0; r < 16; r++) v[r] = part_load(a.part + pidx(sl, i, j, r));
                     tot[i][j] = sl == 0 ? v : tot[i][j] + v;
                 }
         }

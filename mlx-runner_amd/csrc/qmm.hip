@@ -333,20 +333,16 @@ __global__ __launch_bounds__(256, 3) void qmb_kernel(QbDev a) {
             const int t = 4 * q + i;
             if (q >= 2 || t >= T || n >= a.O) continue;
             if (a.S == 1) finish(t, n, sum);
-            else __hip_atomic_store(a.part + ((int64_t)z * T + t) * a.O + n, sum, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            else part_store(a.part + ((int64_t)z * T + t) * a.O + n, sum);
         }
     }
     if (a.S == 1) return;
-    // The partial sums were stored at agent scope (through to memory), and every wave waits for its own before
-    // the counter moves: no cache has to be written back or invalidated, which an acquire-release would do
-    // (4096 -> 4096 in 16 ranges: 37 us with it).
-    __builtin_amdgcn_s_waitcnt(0);
-    __syncthreads();
+    parts_stored();
     __shared__ int last;
-    if (tid == 0) last = __hip_atomic_fetch_add(a.cnt + blk, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == (unsigned)(a.S - 1);
+    if (tid == 0) last = part_last(a.cnt + blk, a.S);
     __syncthreads();
     if (!last) return;
-    if (tid == 0) __hip_atomic_store(a.cnt + blk, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (tid == 0) part_rearm(a.cnt + blk);
     for (int i = tid; i < 64 * RT * T; i += 256) {
         const int n = blk * 64 * RT + i % (64 * RT), t = i / (64 * RT);
         if (n >= a.O) continue;
@@ -355,7 +351,7 @@ __global__ __launch_bounds__(256, 3) void qmb_kernel(QbDev a) {
             float v[8];
 #pragma unroll
             for (int k = 0; k < 8; k++)
-                v[k] = __hip_atomic_load(a.part + ((int64_t)min(y + k, a.S - 1) * T + t) * a.O + n, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                v[k] = part_load(a.part + ((int64_t)min(y + k, a.S - 1) * T + t) * a.O + n);
 #pragma unroll
             for (int k = 0; k < 8; k++)
                 if (y + k < a.S) sum += v[k];
