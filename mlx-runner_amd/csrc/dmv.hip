@@ -568,12 +568,7 @@ bool dpack_mv_supported(const MvPhaseDesc& p) {
 hipError_t launch_dpack_mv(const MvPhaseDesc& p, const float* x, const float* norm_w, float eps, float* y, int mode,
                            hipStream_t s, float* split) {
     if (!dpack_mv_supported(p) || mode < 0 || mode > 2) return hipErrorInvalidValue;
-    static int cus = 0;
-    if (!cus) {
-        int dev = 0;
-        if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
-            return hipErrorInvalidDevice;
-    }
+    const int cus = device_cus();
     // workgroups per CU: 2 (what the registers let run at once), 1 for inputs over 16K values (their
     // f16 hi + lo image alone takes over half the LDS); more only queues extra rounds (measured on
     // the 32B projections: gate|up 43 -> 36 us at 2, down 48 -> 37 us at 1)
@@ -655,12 +650,7 @@ size_t dpack_mm_split_floats(const MvPhaseDesc& p) {
 hipError_t launch_dpack_mm(const MvPhaseDesc& p, const float* x, int xs, const float* norm_w, float eps, float* y, int ys,
                            bool accumulate, int T, float* split, size_t split_floats, hipStream_t s) {
     if (!dpack_mv_supported(p) || T < 1 || T > DMM_TOK || (p.gated && accumulate)) return hipErrorInvalidValue;
-    static int cus = 0;
-    if (!cus) {
-        int dev = 0;
-        if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
-            return hipErrorInvalidDevice;
-    }
+    const int cus = device_cus();
     static bool attr = false;
     if (!attr) {
         for (const void* f : {(const void*)dpack_mm_kernel<4, false, 1>, (const void*)dpack_mm_kernel<8, false, 1>,

@@ -7,7 +7,6 @@
 // and every product accumulates in fp32, so the result matches fp32 arithmetic to ~1e-5 relative.
 //
 #include "kernels.h"
-#include <atomic>
 #include <type_traits>
 
 namespace mlxr {
@@ -267,20 +266,13 @@ __global__ __launch_bounds__(256, 2) void flash_kernel(FlashDev f) {
     }
 }
 
-static int flash_cus() {
-    static std::atomic<int> cus{0};
-    if (int c = cus.load(std::memory_order_relaxed)) return c;
-    int dev = 0, n = 0;
-    if (hipGetDevice(&dev) == hipSuccess && hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && n > 0) cus = n;
-    return n > 0 ? n : 256;
-}
 hipError_t launch_flash_prefill(const FlashArgs& a, hipStream_t s) {
     if (a.D != 128 || a.nKV < 1 || a.nH % a.nKV || a.nH / a.nKV > 8 || a.T < 1) return hipErrorInvalidValue;
     FlashDev f{};
     f.a = a;
     f.nb = (a.T + 31) / 32;
     f.nwg = (a.nH / a.nKV * f.nb + 3) / 4;
-    const int cus = flash_cus(), total = f.nwg * a.nKV;
+    const int cus = device_cus(), total = f.nwg * a.nKV;
     f.first = total > cus && total <= 2 * cus ? cus / a.nKV : f.nwg;
     hipLaunchKernelGGL(flash_kernel, dim3(total), dim3(256), 4 * F2_TILE, s, f);
     return hipGetLastError();

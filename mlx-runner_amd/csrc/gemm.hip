@@ -191,12 +191,7 @@ hipError_t launch_qgemm(const QGemmArgs& a, hipStream_t s) {
     d.w = a.m.w; d.s = direct ? a.m.s : a.wsb; d.b = a.m.b; d.bias = a.m.bias; d.st = a.st; d.direct = direct;
     d.K = a.K; d.O = a.O; d.T = a.T; d.ys = a.y_stride; d.SF = qgemm_slices(a.K, a.O);
     d.xh = a.xbf; d.xl = a.xlo; d.gsum = reinterpret_cast<const uint16_t*>(a.xgs); d.inv = a.xsc; d.nz = a.xnz; d.y = a.y;
-    static int cus = 0;
-    if (!cus) {
-        int dev = 0;
-        if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
-            return hipErrorInvalidDevice;
-    }
+    const int cus = device_cus();
     const bool split = a.split && a.split_floats >= QGEMM_SPLIT_FLOATS;
     const QGemmCut q = qgemm_cut(a.T, a.K, a.O, a.gs, d.SF, cus, split);
     d.S = q.S;

@@ -2,6 +2,7 @@
 // All launchers validate nothing: the callers in model.cpp / capi.cpp check shapes first.
 #pragma once
 #include "common.h"
+#include <atomic>
 
 namespace mlxr {
 
@@ -74,6 +75,17 @@ size_t qgemm_scale_halves(int O, int K, int gs);
 // launch_x_to_f16's single-pass kernel (misc.hip) for K <= 32768; false (nothing launched) above.
 bool launch_row_f16(const float* x, int xs, int K, int T, uint16_t* out, float* inv, hipStream_t s);
 hipError_t launch_x_to_f16(const float* x, int xs, int K, int T, uint16_t* out, float* inv, hipStream_t s);
+
+// The device's compute units, which launches are cut for (256 where there is no device to ask: the launch
+// then says so itself).
+inline int device_cus() {
+    static std::atomic<int> cus{0};
+    if (const int c = cus.load(std::memory_order_relaxed)) return c;
+    int dev = 0, n = 0;
+    if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) return 256;
+    cus = n;
+    return n;
+}
 
 // Embedding: out[t][k] = dequant(row ids[t]) (ids read from hist + *dpos + t0).
 hipError_t launch_qembed(const QMat& m, int K, int bits, int gs, int st, const int* hist, const int* dpos, int T,

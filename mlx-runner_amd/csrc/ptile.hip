@@ -267,15 +267,6 @@ static hipError_t tile_gemm_launch(const TileGemmArgs& a0, hipStream_t s) {
     return hipGetLastError();
 }
 
-static int device_cus() {
-    static int cus = 0;
-    if (!cus) {
-        int dev = 0, n = 0;
-        if (hipGetDevice(&dev) == hipSuccess && hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess) cus = n;
-    }
-    return cus > 0 ? cus : 256;
-}
-
 // The cut with the least expected time. A workgroup of nb blocks takes a + nb * tb microseconds (fill
 // and epilogue, then one 128-k block after another); a CU that is given n of them takes n times that
 // where one fits (16 mi >= 128 tokens), and hides all but e of the next one's a where two do. Measured

@@ -10,10 +10,6 @@ typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
 typedef __bf16 gx_bf8 __attribute__((ext_vector_type(8)));
 typedef uint32_t gx_u4 __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) void* gx_lptr;
-__device__ __forceinline__ uint4 gload_u4(const void* p) {
-    const gx_u4 v = gload(reinterpret_cast<const gx_u4*>(p));
-    return uint4{v.x, v.y, v.z, v.w};
-}
 
 constexpr int GX_K = 64, GX_NST = 3;
 constexpr int GX_RSRC_W3 = 0x00020000;   // raw buffer, 32-bit data format

@@ -24,7 +24,6 @@
 // 4096 -> 14336 at 8 bits 32.7 -> 22.0, 14336 -> 4096 at 6 bits 41.5 -> 20.1, 14336 -> 512 at 4 bits 27.7 -> 10.6,
 // 1024 -> 512 at 4 bits 9.3 -> 7.6; without the exchange 4096 -> 30000 at 3 bits took 33.9, with it 31.
 #include "qgemm.h"
-#include <atomic>
 
 namespace mlxr {
 
@@ -360,14 +359,6 @@ __global__ __launch_bounds__(256, 3) void qmb_kernel(QbDev a) {
     }
 }
 
-static int qb_cus() {
-    static std::atomic<int> cus{0};
-    if (int c = cus.load(std::memory_order_relaxed)) return c;
-    int dev = 0, n = 0;
-    if (hipGetDevice(&dev) == hipSuccess && hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && n > 0) cus = n;
-    return n > 0 ? n : 256;
-}
-
 // The shapes whose x goes to the matrix cores as f16 hi + lo: a value keeps 22 bits beside the largest of its
 // 1024 inputs, fewer the smaller it is beside that, and an infinity comes out as NaN. 5-bit codes, and 2, 3 and
 // 6 bits where K is no whole number of eight groups (four of 128 codes), hold x in fp32 and stay on the vector
@@ -387,7 +378,7 @@ hipError_t launch_qmb(const QmmSmallArgs& a, hipStream_t s) {
     }
     d.o1 = a.part[0].O; d.o2 = a.nparts > 1 ? a.part[1].O : 0;
     d.K = a.K; d.O = a.O; d.T = a.T; d.xs = a.x_stride; d.ys = a.y_stride; d.x = a.x; d.y = a.y;
-    const int C = (a.K + QB_CH - 1) / QB_CH, cus = qb_cus();
+    const int C = (a.K + QB_CH - 1) / QB_CH, cus = device_cus();
     // Tiles per wave and K ranges by expected time: a round of a workgroup per CU takes 2 us to start, 0.3 us a
     // chunk to convert x and 0.7 us a chunk and tile (a CU holds three or four workgroups, so later rounds
     // overlap a little); ranges add the hand-over, more with more partial sums. Over 120 shapes (512 .. 151936 rows,
