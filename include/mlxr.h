@@ -223,15 +223,23 @@ int mlxr_k_qmv(const mlxr_qmat* parts, int nparts, int K, int bits, int gs, int 
 /* Small batch, T in 1..8 (`qmm` / `qmvx4`, Kernels.swift:60-113, 518-622). */
 int mlxr_k_qmm(const mlxr_qmat* parts, int nparts, int K, int bits, int gs, int st, int T, const float* x,
                int x_stride, float* y, int y_stride);
-/* Prefill GEMM on bf16 MFMA (`qgemm`, Kernels.swift:785-851), any T >= 1. */
+/* Prefill GEMM with exact codes, x as an f16 hi + lo pair (`qgemm`, Kernels.swift:785-851), any T >= 1. */
 int mlxr_k_qgemm(const mlxr_qmat* mat, int K, int bits, int gs, int st, int T, const float* x, int x_stride,
                  float* y, int y_stride);
+/* The same under a given cut, for tests: tiles of 128 x 256, 64 x 128 or 32 x 128 (tokens x rows; cut 0, 1, 2),
+ * the K slices over `slices` workgroups per tile. MLXR_E_UNSUPPORTED where the launch could not take it. */
+int mlxr_k_qgemm_cut(const mlxr_qmat* mat, int K, int bits, int gs, int st, int T, const float* x, int x_stride,
+                     float* y, int y_stride, int cut, int slices);
 /* The prefill GEMM over the repacked decode tiles that model prefill uses for 4-bit bf16-scale
  * models (`qgemm`, Kernels.swift:785-851): parts [A|B|C] as in mlxr_k_qmv, bits 4, bf16 scales,
  * gs 32/64, K % 128 == 0; gated (two parts of equal O): y[t][o] = silu(A x_t)[o] * (B x_t)[o]
  * (the MLP's gate|up, silu_mul Kernels.swift:2004-2013). Repacks into a temporary buffer per call. */
 int mlxr_k_qgemm_tiles(const mlxr_qmat* parts, int nparts, int K, int gs, int gated, int T, const float* x,
                        int x_stride, float* y, int y_stride);
+/* The same under a given cut, for tests: 16 mi tokens (mi 1, 2, 4, 8) x 8 rt row tiles (rt 2, or 3 with mi 8)
+ * per workgroup. MLXR_E_UNSUPPORTED for others. */
+int mlxr_k_qgemm_tiles_cut(const mlxr_qmat* parts, int nparts, int K, int gs, int gated, int T, const float* x,
+                           int x_stride, float* y, int y_stride, int mi, int rt);
 /* Batch-1 matvec over the repacked tiles, the kernel-per-op decode step's projection (`qmv` with
  * its fused epilogues, Kernels.swift:60-113, 1037-1070, 2004-2013): mode 0 y = W x (+ bias),
  * 1 y += W x (+ bias), 2 (two parts of equal O) y[o] = silu(A x)[o] * (B x)[o]; norm_w (or NULL)

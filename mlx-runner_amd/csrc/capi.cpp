@@ -252,7 +252,8 @@ int mlxr_k_qmm(const mlxr_qmat* parts, int nparts, int K, int bits, int gs, int 
     return done(launch_qmm_small(a, g_stream));
 }
 
-int mlxr_k_qgemm(const mlxr_qmat* mat, int K, int bits, int gs, int st, int T, const float* x, int x_stride, float* y, int y_stride) {
+static int run_qgemm(const mlxr_qmat* mat, int K, int bits, int gs, int st, int T, const float* x, int x_stride, float* y, int y_stride,
+                     int cut, int slices) {
     std::lock_guard<std::mutex> lk(g_mu);
     if (int rc = ensure_stream()) return rc;
     if (int rc = check_parts(mat, 1)) return rc;
@@ -269,7 +270,18 @@ int mlxr_k_qgemm(const mlxr_qmat* mat, int K, int bits, int gs, int st, int T, c
     a.x = x; a.x_stride = x_stride; a.y = y; a.y_stride = y_stride; a.xbf = g_xbf; a.xsc = g_xsc;
     a.xlo = g_xlo; a.xgs = g_xgs; a.xnz = g_xnz; a.wsb = g_wsb;
     a.split = g_qsplit; a.split_floats = g_qsplit_floats;
-    return done(launch_qgemm(a, g_stream));
+    a.cut = cut; a.slices = slices;
+    const hipError_t e = launch_qgemm(a, g_stream);
+    if (cut >= 0 && e == hipErrorInvalidValue) return set_error(MLXR_E_UNSUPPORTED, "cut");
+    return done(e);
+}
+int mlxr_k_qgemm(const mlxr_qmat* mat, int K, int bits, int gs, int st, int T, const float* x, int x_stride, float* y, int y_stride) {
+    return run_qgemm(mat, K, bits, gs, st, T, x, x_stride, y, y_stride, -1, 0);
+}
+int mlxr_k_qgemm_cut(const mlxr_qmat* mat, int K, int bits, int gs, int st, int T, const float* x, int x_stride, float* y, int y_stride,
+                     int cut, int slices) {
+    if (cut < 0) return set_error(MLXR_E_INVALID_ARG, "cut");
+    return run_qgemm(mat, K, bits, gs, st, T, x, x_stride, y, y_stride, cut, slices);
 }
 
 // Repacks the parts into a temporary DPack (freed by the caller).
@@ -298,8 +310,8 @@ static int tiles_pack(const mlxr_qmat* parts, int nparts, int K, int gs, int gat
     return MLXR_OK;
 }
 
-int mlxr_k_qgemm_tiles(const mlxr_qmat* parts, int nparts, int K, int gs, int gated, int T, const float* x, int x_stride,
-                       float* y, int y_stride) {
+static int run_qgemm_tiles(const mlxr_qmat* parts, int nparts, int K, int gs, int gated, int T, const float* x, int x_stride,
+                           float* y, int y_stride, TilePlan plan) {
     std::lock_guard<std::mutex> lk(g_mu);
     if (int rc = ensure_stream()) return rc;
     int rows = 0;
@@ -311,11 +323,21 @@ int mlxr_k_qgemm_tiles(const mlxr_qmat* parts, int nparts, int K, int gs, int ga
     if (int rc = ensure_buf(g_xbf, g_xbf_elems, (size_t)T * K)) { hipFree(code); return rc; }
     if (int rc = ensure_buf(g_xsc, g_xsc_elems, (size_t)T)) { hipFree(code); return rc; }
     hipError_t e = launch_x_to_f16(x, x_stride, K, T, g_xbf, g_xsc, g_stream);
-    if (e == hipSuccess) e = launch_tile_gemm(d, g_xbf, g_xsc, T, y, y_stride, tile_gemm_plan(d, T), g_stream);
+    if (e == hipSuccess) e = launch_tile_gemm(d, g_xbf, g_xsc, T, y, y_stride, plan.mi ? plan : tile_gemm_plan(d, T), g_stream);
     const hipError_t e2 = hipStreamSynchronize(g_stream);
     hipFree(code);
     if (e == hipSuccess) e = e2;
+    if (plan.mi && e == hipErrorInvalidValue) return set_error(MLXR_E_UNSUPPORTED, "cut");
     return done(e);
+}
+int mlxr_k_qgemm_tiles(const mlxr_qmat* parts, int nparts, int K, int gs, int gated, int T, const float* x, int x_stride,
+                       float* y, int y_stride) {
+    return run_qgemm_tiles(parts, nparts, K, gs, gated, T, x, x_stride, y, y_stride, TilePlan{0, 0});
+}
+int mlxr_k_qgemm_tiles_cut(const mlxr_qmat* parts, int nparts, int K, int gs, int gated, int T, const float* x, int x_stride,
+                           float* y, int y_stride, int mi, int rt) {
+    if (mi < 1) return set_error(MLXR_E_INVALID_ARG, "cut");
+    return run_qgemm_tiles(parts, nparts, K, gs, gated, T, x, x_stride, y, y_stride, TilePlan{mi, rt});
 }
 
 int mlxr_k_qmv_tiles(const mlxr_qmat* parts, int nparts, int K, int gs, int mode, const float* x, const float* norm_w, float eps,

@@ -151,17 +151,22 @@ static int qgemm_slices(int K, int O) {
 // all cuts. 8 bits, 4096 -> 14336, 512 tokens: 128 x 256 unsplit 145 us (64 x 128: 216); 16 tokens: 32 x 128 in two
 // slices 41 us (128 x 256 unsplit 142); 3 bits, 14336 -> 4096, 48 tokens: 64 x 128 in eight 58 us (616).
 struct QGemmCut { int cut, S; };
+struct QGemmKind { int tok, rows; double a, alone, shared; };
+static const QGemmKind qgemm_kinds[] = {{GxBig::TOK, GxBig::NR, 14.0, 2.05, 0.0}, {GxMid::TOK, GxMid::NR, 12.0, 1.3, 1.05},
+                                        {GxSmall::TOK, GxSmall::NR, 9.0, 0.8, 0.88}};
+static size_t qgemm_tiles(const QGemmKind& k, int T, int O) { return (size_t)((T + k.tok - 1) / k.tok) * ((O + k.rows - 1) / k.rows); }
+static bool qgemm_cut_fits(const QGemmKind& k, int T, int O, int SF, int S, bool split) {
+    const size_t tiles = qgemm_tiles(k, T, O);
+    return S == 1 || (S > 1 && S <= SF && split && tiles <= QGEMM_SPLIT_TILES && tiles * SF * k.tok * k.rows <= QGEMM_SPLIT_PART);
+}
 static QGemmCut qgemm_cut(int T, int K, int O, int gs, int SF, int cus, bool split) {
-    struct Kind { int tok, rows; double a, alone, shared; };
-    static const Kind kinds[] = {{GxBig::TOK, GxBig::NR, 14.0, 2.05, 0.0}, {GxMid::TOK, GxMid::NR, 12.0, 1.3, 1.05},
-                                 {GxSmall::TOK, GxSmall::NR, 9.0, 0.8, 0.88}};
     QGemmCut best{0, 1};
     double bt = 1e30;
     for (int c = 0; c < 3; c++)
         for (int S = 1; S <= SF; S++) {
-            const Kind& k = kinds[c];
-            const size_t tiles = (size_t)((T + k.tok - 1) / k.tok) * ((O + k.rows - 1) / k.rows);
-            if (S > 1 && (!split || tiles > QGEMM_SPLIT_TILES || tiles * SF * k.tok * k.rows > QGEMM_SPLIT_PART)) continue;
+            const QGemmKind& k = qgemm_kinds[c];
+            const size_t tiles = qgemm_tiles(k, T, O);
+            if (!qgemm_cut_fits(k, T, O, SF, S, split)) continue;
             const double n = (double)(tiles * S) / cus, blocks = (double)K / GX_K * ((SF + S - 1) / S) / SF * (gs == 32 ? 1.15 : 1.0);
             double t = k.a + blocks * (c == 0 ? (double)((tiles * S + cus - 1) / cus) * k.alone : n * k.shared > k.alone ? n * k.shared : k.alone);
             if (S > 1) t += 6.0 + (double)(tiles * SF * k.tok * k.rows) * 8 / 4e6;
@@ -193,7 +198,9 @@ hipError_t launch_qgemm(const QGemmArgs& a, hipStream_t s) {
     d.xh = a.xbf; d.xl = a.xlo; d.gsum = reinterpret_cast<const uint16_t*>(a.xgs); d.inv = a.xsc; d.nz = a.xnz; d.y = a.y;
     const int cus = device_cus();
     const bool split = a.split && a.split_floats >= QGEMM_SPLIT_FLOATS;
-    const QGemmCut q = qgemm_cut(a.T, a.K, a.O, a.gs, d.SF, cus, split);
+    QGemmCut q{a.cut, a.slices};
+    if (a.cut < 0) q = qgemm_cut(a.T, a.K, a.O, a.gs, d.SF, cus, split);
+    else if (a.cut > 2 || !qgemm_cut_fits(qgemm_kinds[a.cut], a.T, a.O, d.SF, a.slices, split)) return hipErrorInvalidValue;
     d.S = q.S;
     if (q.S > 1) { d.cnt = reinterpret_cast<unsigned*>(a.split); d.part = a.split + QGEMM_SPLIT_TILES; }
     switch (a.bits) {

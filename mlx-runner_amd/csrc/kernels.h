@@ -62,6 +62,7 @@ struct QGemmArgs {
     // optional scratch for K slices on workgroups of their own: QGEMM_SPLIT_FLOATS floats, zero before
     // first use (its tile counters return to zero)
     float* split = nullptr; size_t split_floats = 0;
+    int cut = -1, slices = 0;             // a given cut (tile shape 0 .. 2, workgroups per tile) instead of the launch's choice
 };
 // tile counters, then the slices' partial tiles (512 of 128 x 256, or as many smaller ones as fit)
 constexpr size_t QGEMM_SPLIT_TILES = 4096, QGEMM_SPLIT_PART = 512 * 128 * 256;

@@ -96,7 +96,9 @@ def _load():
         "mlxr_k_qmv": (I, [C.POINTER(QMat), I, I, I, I, I, P, P, F, P, I]),
         "mlxr_k_qmm": (I, [C.POINTER(QMat), I, I, I, I, I, I, P, I, P, I]),
         "mlxr_k_qgemm": (I, [C.POINTER(QMat), I, I, I, I, I, P, I, P, I]),
+        "mlxr_k_qgemm_cut": (I, [C.POINTER(QMat), I, I, I, I, I, P, I, P, I, I, I]),
         "mlxr_k_qgemm_tiles": (I, [C.POINTER(QMat), I, I, I, I, I, P, I, P, I]),
+        "mlxr_k_qgemm_tiles_cut": (I, [C.POINTER(QMat), I, I, I, I, I, P, I, P, I, I, I]),
         "mlxr_k_qmv_tiles": (I, [C.POINTER(QMat), I, I, I, I, P, P, C.c_float, P, I]),
         "mlxr_k_qmm_tiles": (I, [C.POINTER(QMat), I, I, I, I, I, P, I, P, F, P, I]),
         "mlxr_k_qembed": (I, [C.POINTER(QMat), I, I, I, I, P, I, P]),

@@ -275,9 +275,9 @@ def test_qgemm_prefill_tiles(gpu, bits, gs):
 @pytest.mark.parametrize("gs", [32, 64, 128])
 @pytest.mark.parametrize("bits", [2, 3, 4, 5, 6, 8])
 def test_qgemm_cuts(gpu, bits, gs):
-    """The MLX-layout GEMM's tile shapes and K slices around their edges (32 / 64 / 128 tokens, 128 / 256
-    rows; 2176 inputs: two slices, a group count that is odd at gs 128; 8320: eight, of uneven length):
-    each T against the fp64 product at the gate, its rows bit-identical to those of the largest T."""
+    """The MLX-layout GEMM as the launch cuts it (test_qgemm_given_cuts runs every cut) over ragged batches
+    (2176 inputs: two slices, a group count that is odd at gs 128; 8320: eight, of uneven length): the
+    largest against the fp64 product at the gate, the others' rows bit-identical to its."""
     for O, K in ((300, 2176), (129, 8320)):
         fx = QuantFixture(O, K, bits, gs, seed=bits + gs, fast=True)
         x = np.random.default_rng(gs + bits).uniform(-1, 1, (200, K)).astype(np.float32)
@@ -286,6 +286,40 @@ def test_qgemm_cuts(gpu, bits, gs):
         assert max_rel_err(full, ref) < TOL, (O, K)
         for T in (9, 32, 33, 65, 129):
             assert np.array_equal(qgemm(gpu, fx, x[:T]).view(np.uint32), full[:T].view(np.uint32)), (T, O, K)
+
+
+@pytest.mark.parametrize("gs", [32, 64, 128])
+@pytest.mark.parametrize("bits", [2, 3, 4, 5, 6, 8])
+def test_qgemm_given_cuts(gpu, bits, gs):
+    """Every tile shape (128 x 256, 64 x 128, 32 x 128) with its K slices on one workgroup (running sums parked in
+    y), on some and on one each: every row bit-identical, ragged tokens and rows, padded output rows, biases,
+    fp32 and bf16-valued inputs (no lo parts); one, two and eight slices of uneven length. Against the fp64
+    product at about four times the relative 2-norm measured (2 bits 3.7e-5, half as much for each further bit:
+    a code enters as q * 2^-24, and the matrix cores align a step's products to its largest, x's lo parts last)."""
+    for O, K, slices in ((300, 2176, 2), (129, 8320, 8), (517, 1152, 1)):
+        fx = QuantFixture(O, K, bits, gs, st="f16" if gs == 64 else "bf16", seed=bits + gs, with_bias=True, fast=True)
+        qm = (gpu.QMat * 1)(fx.device(gpu))
+        for T, bf16_x in ((150, False), (9, True)):
+            x = np.random.default_rng(gs + bits).normal(0, 1, (T, K)).astype(np.float32)
+            if bf16_x:
+                x = bf16_to_f32(bf16_round(x)).reshape(T, K)
+            dx, first = gpu.DeviceArray.from_numpy(x), None
+            for cut in range(3):
+                for S in range(1, slices + 2):
+                    dy = gpu.DeviceArray.from_numpy(np.full((T, O + 3), np.nan, np.float32))
+                    rc = gpu.lib.mlxr_k_qgemm_cut(qm, K, bits, gs, int(gs == 64), T, dx.ptr, K, dy.ptr, O + 3, cut, S)
+                    if S > slices:
+                        assert rc == -4, rc
+                        continue
+                    gpu.check(rc)
+                    gpu.synchronize()
+                    got = dy.numpy()
+                    assert np.all(np.isnan(got[:, O:]))
+                    if first is None:
+                        first = got[:, :O]
+                    assert np.array_equal(got[:, :O].view(np.uint32), first.view(np.uint32)), (O, K, T, cut, S)
+            ref = fx.oracle(oracle).matmul_f64(x).astype(np.float64)
+            assert np.linalg.norm(first - ref) <= 1.2e-3 * 2.0**-bits * np.linalg.norm(ref), (O, K, T)
 
 
 def test_qgemm_pointer_alignment(gpu):
@@ -340,7 +374,7 @@ def qgemm_tiles(mlxr, fxs, x, gated=False):
 def test_qgemm_tiles(gpu, gs):
     """The prefill GEMM over repacked tiles (model prefill's path for 4-bit bf16-scale models):
     fused parts [A|B|C] with per-part bias (or none) and ragged row counts, against the oracle's 4-bit GEMM
-    precision per part; T not a multiple of the 128-token tile."""
+    precision per part; ragged T, as the launch cuts it (test_qgemm_tiles_given_cuts runs every cut)."""
     K = 512
     for T in (9, 130, 300):
         fxs = [QuantFixture(O, K, 4, gs, seed=O + T, with_bias=T != 130, fast=True) for O in (264, 40, 88)]
@@ -349,6 +383,38 @@ def test_qgemm_tiles(gpu, gs):
         ref = np.concatenate([f.oracle(oracle).matmul_f16(x) for f in fxs], axis=1)
         assert max_rel_err(got, ref) < TOL, T
         assert np.max(np.abs(got - ref)) < 1e-4, T
+
+
+@pytest.mark.parametrize("gs", [32, 64])
+@pytest.mark.parametrize("K", [128, 256, 384, 1152])
+def test_qgemm_tiles_given_cuts(gpu, gs, K):
+    """Every cut of the tile GEMM (16 / 32 / 64 / 128 tokens x 16 row tiles, 128 x 24) over K of one block, fewer
+    blocks than copy stages, and more; tokens and rows that are no multiple of a workgroup's, three parts with
+    bias, gate | up: the first against the oracle's GEMM precision, all others bit-identical to it."""
+    def run(fxs, x, gated, mi, rt):
+        T, O = x.shape[0], fxs[0].O if gated else sum(f.O for f in fxs)
+        qm = (gpu.QMat * len(fxs))(*[f.device(gpu) for f in fxs])
+        dx, dy = gpu.DeviceArray.from_numpy(x), gpu.DeviceArray.from_numpy(np.full((T, O + 1), np.nan, np.float32))
+        gpu.check(gpu.lib.mlxr_k_qgemm_tiles_cut(qm, len(fxs), K, gs, int(gated), T, dx.ptr, K, dy.ptr, O + 1, mi, rt))
+        gpu.synchronize()
+        got = dy.numpy()
+        assert np.all(np.isnan(got[:, O:]))
+        return got[:, :O]
+    for T in (1, 33, 150):
+        x = np.random.default_rng(T).normal(0, 1, (T, K)).astype(np.float32)
+        for gated, Os in ((False, (264, 43, 88)), (True, (203, 203))):
+            fxs = [QuantFixture(O, K, 4, gs, seed=O + T + i, with_bias=True, fast=True) for i, O in enumerate(Os)]
+            first = run(fxs, x, gated, 8, 2)
+            refs = [f.oracle(oracle).matmul_f16(x) for f in fxs]
+            if gated:
+                ref = (refs[0] / (1.0 + np.exp(-refs[0].astype(np.float64)))).astype(np.float32) * refs[1]
+            else:
+                ref = np.concatenate(refs, axis=1)
+            assert max_rel_err(first, ref) < TOL, (T, gated)
+            for mi, rt in ((1, 2), (2, 2), (4, 2), (8, 3)):
+                assert np.array_equal(run(fxs, x, gated, mi, rt).view(np.uint32), first.view(np.uint32)), (T, gated, mi, rt)
+    with pytest.raises(gpu.EngineError):
+        run(fxs, x, True, 4, 3)
 
 
 @pytest.mark.parametrize("gs", [32, 64])
@@ -589,11 +655,10 @@ def test_qgemm_batch_invariant(gpu):
 
 @pytest.mark.parametrize("bits,gs", [(3, 32), (8, 64)])
 def test_qgemm_split_k_batch_invariant(gpu, bits, gs):
-    """The MLX-layout GEMM over a long input (128 K steps: four fixed K slices added in order):
-    a launch of few tiles runs the slices on workgroups of their own (9 tokens x 40 row tiles), a
-    launch of many does not (512 tokens x 40), and a token's result is bit-identical either way
-    (prefillTilesAgreeBitwise, KernelTests.swift:168-184), and matches the fp64 product at the
-    1e-3 gate; repeated, so the split's tile counters are back at zero."""
+    """The MLX-layout GEMM over a long input (128 K steps, six fixed K slices added in order): 9 and 512
+    tokens spread the slices over different numbers of workgroups in tiles of different shapes, and a
+    token's result is bit-identical either way (prefillTilesAgreeBitwise, KernelTests.swift:168-184), and
+    matches the fp64 product at the 1e-3 gate; repeated, so the tile counters are back at zero."""
     O, K = 5120, 8192
     fx = QuantFixture(O, K, bits, gs, seed=bits, fast=True)
     x = np.random.default_rng(bits).uniform(-1, 1, (512, K)).astype(np.float32)
