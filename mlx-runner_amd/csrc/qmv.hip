@@ -161,25 +161,28 @@ __global__ __launch_bounds__(256) void qmv_kernel(QmvDev a) {
     for (int r = 0; r < R; r++) acc[r] = 0.0f;
     const int nchunks = K >> 5;
     const int cq0 = KS ? nchunks * wave / QMV_WAVES : 0, cq1 = KS ? nchunks * (wave + 1) / QMV_WAVES : nchunks;
-    auto chunk = [&](int c, const uint32_t (&w)[R][BITS], const uint16_t (&s)[R], const uint16_t (&b)[R]) {
-        float x[32];
-#pragma unroll
-        for (int i = 0; i < 8; i++) {
-            const float4 v = *reinterpret_cast<const float4*>(xsrc + (c << 5) + 4 * i);
-            x[4 * i] = v.x; x[4 * i + 1] = v.y; x[4 * i + 2] = v.z; x[4 * i + 3] = v.w;
-        }
-        float xsum = 0.0f;
-#pragma unroll
-        for (int j = 0; j < 32; j++) xsum += x[j];
-#pragma unroll
-        for (int r = 0; r < R; r++) acc[r] += ld_scale<ST>(&s[r]) * chunk_dot<BITS>(w[r], x) + ld_scale<ST>(&b[r]) * xsum;
-    };
-    auto fetch = [&](int c, uint32_t (&w)[R][BITS], uint16_t (&s)[R], uint16_t (&b)[R]) {
-        const int g = (c << 5) / a.gs;
-#pragma unroll
-        for (int r = 0; r < R; r++) { load_chunk<BITS>(wp[r] + (int64_t)c * (4 * BITS), w[r]); s[r] = sp[r][g]; b[r] = bp[r][g]; }
-    };
     if constexpr (KS == 2) {
+        auto fetch = [&](int c, uint32_t (&w)[R][BITS], uint16_t (&s)[R], uint16_t (&b)[R]) {
+            const int g = (c << 5) / a.gs;
+#pragma unroll
+            for (int r = 0; r < R; r++) { load_chunk<BITS>(wp[r] + (int64_t)c * (4 * BITS), w[r]); s[r] = sp[r][g]; b[r] = bp[r][g]; }
+        };
+        auto chunk = [&](int c, const uint32_t (&w)[R][BITS], const uint16_t (&s)[R], const uint16_t (&b)[R]) {
+            float x[32], xsum = 0.0f;
+#pragma unroll
+            for (int i = 0; i < 8; i++) {
+                const float4 v = *reinterpret_cast<const float4*>(xsrc + (c << 5) + 4 * i);
+                x[4 * i] = v.x; x[4 * i + 1] = v.y; x[4 * i + 2] = v.z; x[4 * i + 3] = v.w;
+            }
+#pragma unroll
+            for (int j = 0; j < 32; j++) xsum += x[j];
+#pragma unroll
+            for (int r = 0; r < R; r++) {   // (in the other loop's terms: the same contractions, the same bits)
+                const float sv = ld_scale<ST>(&s[r]), bv = ld_scale<ST>(&b[r]);
+                const float d = chunk_dot<BITS>(w[r], x);
+                acc[r] += sv * d + bv * xsum;
+            }
+        };
         uint32_t w0[R][BITS], w1[R][BITS];
         uint16_t s0[R], b0[R], s1[R], b1[R];
         for (int c = cq0 + lane; c < cq1; c += 128) {
@@ -191,11 +194,28 @@ __global__ __launch_bounds__(256) void qmv_kernel(QmvDev a) {
             if (two) chunk(c + 64, w1, s1, b1);
         }
     } else {
+        // (written out: through functions shared with the loop above, 2-bit rows took 3 to 5% more)
         for (int c = cq0 + lane; c < cq1; c += 64) {
+            const int k0 = c << 5;
             uint32_t w[R][BITS];
-            uint16_t s[R], b[R];
-            fetch(c, w, s, b);
-            chunk(c, w, s, b);
+#pragma unroll
+            for (int r = 0; r < R; r++) load_chunk<BITS>(wp[r] + (int64_t)c * (4 * BITS), w[r]);
+            float x[32];
+#pragma unroll
+            for (int i = 0; i < 8; i++) {
+                const float4 v = *reinterpret_cast<const float4*>(xsrc + k0 + 4 * i);
+                x[4 * i] = v.x; x[4 * i + 1] = v.y; x[4 * i + 2] = v.z; x[4 * i + 3] = v.w;
+            }
+            float xsum = 0.0f;
+#pragma unroll
+            for (int j = 0; j < 32; j++) xsum += x[j];
+            const int g = k0 / a.gs;
+#pragma unroll
+            for (int r = 0; r < R; r++) {
+                const float s = ld_scale<ST>(sp[r] + g), b = ld_scale<ST>(bp[r] + g);
+                const float d = chunk_dot<BITS>(w[r], x);
+                acc[r] += s * d + b * xsum;
+            }
         }
     }
 #pragma unroll
@@ -276,14 +296,16 @@ hipError_t launch_qmv(const QmvArgs& a, hipStream_t s) {
     const int rows = split ? QMV_KS_ROWS : QMV_ROWS;
     const int per_wg = (split ? 1 : QMV_WAVES) * (a.epi == EPI_GATED ? rows / 2 : rows);
     const int grid = (a.O + per_wg - 1) / per_wg;
-    // Such a wave has one to a few chunks a lane, and each was a round trip to memory of its own. Two chunks
-    // in flight cost registers (6 bits: 228, two workgroups per CU), which tells where many rounds of
-    // workgroups hide the round trips: so where the launch is short, or the waves have two chunks of wide
-    // codes, or more than two of any. us per launch, one -> two chunks: 14336 -> 4096 at 3 / 4 / 6 bits 14.2 ->
-    // 13.9, 15.9 -> 15.1, 19.3 -> 17.6; 14336 -> 8192 6 bits 30.2 -> 28.0; 14336 -> 28672 6 bits 111 -> 82;
-    // 27648 -> 16384 5 bits 122 -> 90; 27648 -> 32768 2 bits 130 -> 108; but 14336 -> 12288 3 bits 32.6 -> 33.8,
-    // 14336 -> 28672 4 bits 66.0 -> 66.4 and 8192 -> 28672 6 bits 43.7 -> 49.6.
-    const bool two = grid <= 1024 || (a.bits >= 5 && a.K > 8192) || a.K > 16384;
+    // Such a wave has one to a few chunks a lane (K / 8192), and each was a round trip to memory of its own. Two
+    // chunks in flight cost registers (2 / 3 / 4 / 6 bits: 161, 184, 191, 229 instead of 79 .. 93: half the workgroups
+    // per CU), which tells where many rounds of workgroups hide the round trips, the more the fewer bytes a chunk
+    // has. Measured at 8192 .. 27648 inputs and 512 .. 40960 rows, matrices from memory, time with two as a share of
+    // that with one: in launches of at most two workgroups a CU 0.70 .. 0.92 at 5 and 6 bits and 0.81 .. 1.01 at 4, at 3
+    // bits 0.89 .. 1.00 from 18432 inputs on but up to 1.05 below, at 2 bits up to 1.12 below 24576. In longer ones at 5
+    // and 6 bits 0.66 .. 1.06 (mean 0.85) from 14336 inputs on but up to 1.20 below, at 4 bits 0.68 .. 1.04 (mean 0.86)
+    // from 20480 on but up to 1.17 below, at 3 bits up to 1.32, at 2 bits 0.77 .. 1.00 from 24576 on.
+    const bool few = grid <= 512;
+    const bool two = a.bits >= 5 ? few || a.K >= 14336 : a.bits == 4 ? few || a.K >= 20480 : a.bits == 3 ? few && a.K >= 18432 : a.K >= 24576;
     const int ks = !split ? 0 : two ? 2 : 1;
     const bool xn = a.norm_w != nullptr;
     const size_t lds = xn ? (size_t)a.K * sizeof(float) : 0;

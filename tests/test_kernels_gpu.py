@@ -59,11 +59,12 @@ def test_qmv_partial_passes(gpu, K):
 
 
 @pytest.mark.parametrize("bits,K,gs,O", [(4, 8192, 64, 20), (3, 8256, 32, 9), (6, 14336, 128, 33), (2, 16448, 32, 8), (5, 25600, 64, 17),
-                                         (4, 8256, 32, 8201), (5, 8192, 64, 8193), (6, 8256, 32, 8195)])
+                                         (4, 8256, 32, 8201), (5, 8192, 64, 8193), (6, 8256, 32, 8195), (2, 24640, 32, 8), (3, 18496, 64, 9),
+                                         (6, 14400, 32, 4099)])
 def test_qmv_split_k(gpu, bits, K, gs, O):
     """Rows whose K is split over a workgroup's waves, one or two chunks of 32 codes in flight per lane: one
-    chunk a lane, a ragged second, a third, rows that end inside a workgroup of eight, and launches past
-    1024 workgroups (one chunk in flight, or two for wide codes over more than one chunk). The bound is the
+    chunk a lane, a ragged second, a third and fourth, rows that end inside a workgroup of eight, and launches
+    past 512 workgroups; every width but 8 bits with one and with two in flight. The bound is the
     arithmetic's, elementwise: a product passes through at most 64 fp32 roundings (32 in its chunk, the group's
     scale and bias, the lane's chunks, the tree over lanes, the waves), each 2^-24 of the row's sum of |terms|.
     The accumulate, fused norm and gated epilogues on the small launches."""
