@@ -138,10 +138,15 @@ bool qgemm_supported(int K, int gs) { return K % GX_K == 0 && (gs == 32 || gs ==
 // Fixed K slices of a matrix: a function of its sizes alone, so a token's result never depends on T or on
 // the launch's cut. As many as give a launch of few tokens a workgroup per CU (32 tokens x 128 rows), of at
 // least 1024 inputs: a launch that walks them itself parks its running sum in y (3 us a slice and 8 bytes
-// per output at 8 TB/s), so wide matrices, which need none for that, get none.
+// per output at 8 TB/s), so wide matrices, which need none for that, get none. No five or seven: a launch of
+// middling T spreads them evenly over two, three or four workgroups a tile. From 8192 inputs on four or eight,
+// unless wide: 27648 -> 16384 at 96 tokens takes 271 us in four slices, 427 in two; 27648 -> 7168 at 256 252 and, in
+// five, 357; 27648 -> 4800 at 384 258 and, in six, 316 (4 bits).
 static int qgemm_slices(int K, int O) {
-    const int want = (33000 + O / 2) / O, most = K / 1024 < 8 ? K / 1024 : 8;
-    return want < 1 || most < 1 ? 1 : want < most ? want : most;
+    const int want = (33000 + O / 2) / O;
+    if (K >= 8192) return want >= 8 ? 8 : want >= 2 ? 4 : 1;
+    const int n = want < K / 1024 ? want : K / 1024;
+    return n < 1 ? 1 : n == 5 || n == 7 ? n - 1 : n;
 }
 
 // The launch's tile shape and the workgroups per tile its slices are spread over, by expected time.

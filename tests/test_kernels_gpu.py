@@ -656,9 +656,8 @@ def test_qgemm_batch_invariant(gpu):
 
 @pytest.mark.parametrize("bits,gs", [(3, 32), (8, 64)])
 def test_qgemm_split_k_batch_invariant(gpu, bits, gs):
-    """The MLX-layout GEMM over a long input (128 K steps, six fixed K slices added in order): 9 and 512
-    tokens spread the slices over different numbers of workgroups in tiles of different shapes, and a
-    token's result is bit-identical either way (prefillTilesAgreeBitwise, KernelTests.swift:168-184), and
+    """The MLX-layout GEMM over a long input (128 K steps, four fixed K slices added in order): 9 and 512
+    tokens run in tiles of different shapes and spread the slices differently, and a token's result is bit-identical either way (prefillTilesAgreeBitwise, KernelTests.swift:168-184), and
     matches the fp64 product at the 1e-3 gate; repeated, so the tile counters are back at zero."""
     O, K = 5120, 8192
     fx = QuantFixture(O, K, bits, gs, seed=bits, fast=True)
