@@ -14,7 +14,7 @@
 // - The bias terms sum_g b[n][g] xsum[m][g] (xsum: the group's sum of scaled x, from the pre-pass)
 //   go through the matrix cores too, 4 groups at a time, straight into tot: xsum as three bf16
 //   parts and b as one (bf16 biases) or two (f16) bf16 parts, every product exact in fp32.
-// - K is summed in fixed slices (qgemm_slices: a function of K alone), added in order, so a token's
+// - K is summed in fixed slices (qgemm_slices: a function of K and O alone), added in order, so a token's
 //   result depends neither on T nor on how the launch is cut.
 // - The row is multiplied back by 2^-e at the end.
 //
