@@ -137,12 +137,10 @@ def test_qmm_small_batch(gpu, bits):
                                          (8, 128, "bf16"), (2, 64, "bf16"), (3, 32, "bf16"), (3, 128, "f16"), (6, 64, "f16"),
                                          (6, 128, "bf16")])
 def test_qmm_small_batch_wide_loads(gpu, bits, gs, st):
-    """The small-batch kernel with wide code loads (32 codes per lane at 2 / 3 / 4 / 6 bits, 16 at 8;
-    several groups per load at gs 32 / 64: one MFMA set per group, the other groups' lanes zeroed;
-    3- and 6-bit codes straddling dwords): K of several batches per wave (the
-    eight-wave launch at 4096 / gs 32), two fused parts with ragged row counts, f16 and bf16
-    scales, T = 1..8 with fp32 inputs (x lo parts in use) and bf16-valued inputs (no lo parts);
-    1e-3 against the fp64 product. 8-bit gs 128 runs the per-group kernel."""
+    """The small batch on the matrix cores (codes of 64 inputs per lane and load, one or two groups of them, or
+    half of one; 3- and 6-bit codes straddling dwords; at 2048 and 4096 inputs several K ranges): two fused
+    parts with ragged row counts, f16 and bf16 scales, T = 1..8 with fp32 inputs (x lo parts in use) and
+    bf16-valued inputs (no lo parts); 1e-3 against the fp64 product."""
     K = 4096 if gs == 32 else 2048
     fa = QuantFixture(40, K, bits, gs, st=st, seed=K + bits, fast=True)
     fb = QuantFixture(27, K, bits, gs, st=st, seed=K + bits + 1, fast=True)
